@@ -54,8 +54,9 @@ __global__ void __launch_bounds__(256) k_gs3d_fwd(GridArgs g, const int64_t* ind
     }
 }
 
-// Backward: grid gradient with float atomics (like the reference, IndirectGridSample3D.cu:691-698) and the uv
-// gradient with the reference's product order (:752-790).
+// Backward for any strides: one thread per sample, the grid gradient with one float atomic per corner and channel (as
+// the reference, IndirectGridSample3D.cu:691-698) and the uv gradient with the reference's product order (:752-790).
+// Channels-last gradients take k_gs3d_bwd_cl below, whose atomics coalesce.
 __global__ void __launch_bounds__(256) k_gs3d_bwd(GridArgs g, const int64_t* index, const float* uv, int64_t S,
                                                   const float* grad_out, float* grad_grid, float* grad_uv)
 {
@@ -122,6 +123,139 @@ __global__ void __launch_bounds__(256) k_gs3d_bwd(GridArgs g, const int64_t* ind
     }
 }
 
+// Backward for a channels-last grid and gradient (channel stride 1, C a multiple of CL).
+//
+// What bounds the scatter is the number of atomic requests, not their bytes: one thread per sample issues C * 8
+// atomics whose 64 lanes all hit different lines. Here 2 CL lanes hold the CL consecutive channels of the two corners
+// of an x edge, which are neighbours in memory, so an atomic instruction makes 32 / CL requests of 8 CL contiguous
+// bytes; and a lane group walks a run of `run` consecutive samples, keeping the current trilinear cell's corner sums
+// in registers and adding them to memory only when the run leaves the cell (samples of a ray stay in a cell for about
+// 4 steps; samples in any other order only merge less). The uv gradient runs first, one thread per sample: the 8
+// corners' channel products are summed into one value per corner, of which the three derivatives are 12 terms each;
+// the coordinates stay in LDS for the walk.
+//
+// Measured on 13.0 M samples of cone-beam rays through 4096 grids of 17^3 x 8, with the uv gradient: 37.0 ms with one
+// thread per sample, 2.7 ms with groups of 8 lanes for one corner, 2.03 ms like this (the bytes alone, 1.3 GB, would
+// take about 0.25 ms; the atomic requests are what is left). Runs of at most 16 / 32 / 64 samples: 2.06 / 2.03 / 2.04.
+constexpr int kGsThreads = 256;
+constexpr int kGsRun     = 32;   // samples of a lane group, at most
+constexpr int kGsTile    = kGsThreads / 8 * kGsRun;  // samples of a block, at most (groups of 8 lanes: CL = 4)
+
+template <int CL>
+__global__ void __launch_bounds__(kGsThreads) k_gs3d_bwd_cl(GridArgs g, const int64_t* __restrict__ index,
+                                                            const float* __restrict__ uv, int64_t S, int32_t run,
+                                                            bool vec4, const float* __restrict__ grad_out,
+                                                            float* __restrict__ grad_grid, float* __restrict__ grad_uv)
+{
+    __shared__ float s_x[3][kGsTile];  // grid coordinates
+    __shared__ int32_t s_n[kGsTile];   // slot, -1: outside the grid
+    const int32_t tile = kGsThreads / (2 * CL) * run;
+    const int64_t i0   = (int64_t)blockIdx.x * tile;
+    const int32_t ns = (int32_t)min<int64_t>(tile, S - i0);
+    for (int32_t j = threadIdx.x; j < ns; j += kGsThreads)
+    {
+        const int64_t i = i0 + j;
+        const int64_t n = index[i];
+        const bool in   = n >= 0 && n < g.N;
+        s_n[j]          = in ? (int32_t)n : -1;
+        if (!in)
+        {
+            if (grad_uv) grad_uv[3 * i] = grad_uv[3 * i + 1] = grad_uv[3 * i + 2] = 0.f;
+            continue;
+        }
+        const Tri t = trilinear(g, n, uv[3 * i], uv[3 * i + 1], uv[3 * i + 2]);
+        s_x[0][j]   = t.ix;
+        s_x[1][j]   = t.iy;
+        s_x[2][j]   = t.iz;
+        if (!grad_uv) continue;
+        float d[8] = {};
+        for (int c = 0; c < g.C; c += 4)
+        {
+            float go[4];
+            if (vec4)
+            {
+                const float4 v = *reinterpret_cast<const float4*>(grad_out + i * g.C + c);
+                go[0] = v.x; go[1] = v.y; go[2] = v.z; go[3] = v.w;
+            }
+            else
+            {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) go[q] = grad_out[i * g.C + c + q];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+            {
+                float v[4];
+                if (vec4)
+                {
+                    const float4 f = *reinterpret_cast<const float4*>(g.grid + t.off[k] + c);
+                    v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+                }
+                else
+                {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] = g.grid[t.off[k] + c + q];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) d[k] = fmaf(v[q], go[q], d[k]);
+            }
+        }
+        const float fx1 = t.ix - (float)t.x0, fx0 = (float)(t.x0 + 1) - t.ix;
+        const float fy1 = t.iy - (float)t.y0, fy0 = (float)(t.y0 + 1) - t.iy;
+        const float fz1 = t.iz - (float)t.z0, fz0 = (float)(t.z0 + 1) - t.iz;
+        // corner k takes the upper neighbour on x / y / z iff bit 0 / 1 / 2 of k is set
+        const float gx = ((d[1] - d[0]) * fy0 + (d[3] - d[2]) * fy1) * fz0 +
+                         ((d[5] - d[4]) * fy0 + (d[7] - d[6]) * fy1) * fz1;
+        const float gy = ((d[2] - d[0]) * fx0 + (d[3] - d[1]) * fx1) * fz0 +
+                         ((d[6] - d[4]) * fx0 + (d[7] - d[5]) * fx1) * fz1;
+        const float gz = ((d[4] - d[0]) * fx0 + (d[5] - d[1]) * fx1) * fy0 +
+                         ((d[6] - d[2]) * fx0 + (d[7] - d[3]) * fx1) * fy1;
+        grad_uv[3 * i + 0] = gx * (float)(g.X - 1) / 2;
+        grad_uv[3 * i + 1] = gy * (float)(g.Y - 1) / 2;
+        grad_uv[3 * i + 2] = gz * (float)(g.Z - 1) / 2;
+    }
+    if (!grad_grid) return;
+    __syncthreads();
+    const int32_t ch = threadIdx.x % CL, xb = (threadIdx.x / CL) & 1;
+    const int32_t j0 = (int32_t)(threadIdx.x / (2 * CL)) * run, j1 = min(ns, j0 + run);
+    for (int32_t c = ch; c < g.C; c += CL)
+    {
+        float acc[4];  // corners (y0, z0), (y1, z0), (y0, z1), (y1, z1) of this lane's x and channel
+        int32_t cn = -1, cx = 0, cy = 0, cz = 0;  // the cell whose sums acc holds (cn < 0: none)
+        auto flush = [&]() {
+            float* base = grad_grid + cn * g.s0 + clip_i(cx + xb, g.X) * g.s4 + c;
+            const int64_t oy[2] = {clip_i(cy, g.Y) * g.s3, clip_i(cy + 1, g.Y) * g.s3};
+            const int64_t oz[2] = {clip_i(cz, g.Z) * g.s2, clip_i(cz + 1, g.Z) * g.s2};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) atomicAdd(base + oz[k >> 1] + oy[k & 1], acc[k]);
+        };
+        for (int32_t j = j0; j < j1; ++j)
+        {
+            const int32_t n = s_n[j];
+            if (n < 0) continue;
+            const float ix = s_x[0][j], iy = s_x[1][j], iz = s_x[2][j];
+            const float go = grad_out[(i0 + j) * g.C + c];
+            const int32_t x0 = (int)floorf(ix), y0 = (int)floorf(iy), z0 = (int)floorf(iz);
+            if (n != cn || x0 != cx || y0 != cy || z0 != cz)
+            {
+                if (cn >= 0) flush();
+                cn = n;
+                cx = x0;
+                cy = y0;
+                cz = z0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) acc[k] = 0.f;
+            }
+            const float fx    = xb ? ix - (float)x0 : (float)(x0 + 1) - ix;
+            const float fy[2] = {(float)(y0 + 1) - iy, iy - (float)y0};
+            const float fz[2] = {(float)(z0 + 1) - iz, iz - (float)z0};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[k] += fx * fy[k & 1] * fz[k >> 1] * go;
+        }
+        if (cn >= 0) flush();
+    }
+}
+
 }  // namespace neat
 
 using namespace neat;
@@ -171,7 +305,24 @@ extern "C"
         NEAT_REQUIRE(S >= 0, "num_samples < 0");
         if (S == 0) return NEAT_OK;
         NEAT_REQUIRE(index && uv && grad_out, "neat_gs3d_bwd: null pointer");
-        k_gs3d_bwd<<<grid_for(S, 256), 256, 0, as_stream(stream)>>>(g, index, uv, S, grad_out, grad_grid, grad_uv);
+        hipStream_t s = as_stream(stream);
+        if (g.s1 == 1 && C % 4 == 0 && N < INT32_MAX)
+        {
+            // lane groups for 8 (or 4) consecutive channels; runs of up to 32 samples while 2048 blocks remain
+            const int32_t CL = C % 8 == 0 ? 8 : 4, groups = kGsThreads / (2 * CL);
+            int32_t run      = 4;
+            while (run < kGsRun && S >= (int64_t)2048 * groups * run * 2) run *= 2;
+            const unsigned nb   = (unsigned)((S + (int64_t)groups * run - 1) / ((int64_t)groups * run));
+            const bool vec4     = channels_last(g) && (reinterpret_cast<uintptr_t>(grad_out) % 16) == 0;
+            if (CL == 8)
+                k_gs3d_bwd_cl<8><<<nb, kGsThreads, 0, s>>>(g, index, uv, S, run, vec4, grad_out, grad_grid, grad_uv);
+            else
+                k_gs3d_bwd_cl<4><<<nb, kGsThreads, 0, s>>>(g, index, uv, S, run, vec4, grad_out, grad_grid, grad_uv);
+        }
+        else
+        {
+            k_gs3d_bwd<<<grid_for(S, 256), 256, 0, s>>>(g, index, uv, S, grad_out, grad_grid, grad_uv);
+        }
         NEAT_LAUNCHED();
         return NEAT_OK;
     }
