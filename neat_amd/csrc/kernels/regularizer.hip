@@ -109,6 +109,7 @@ __device__ __forceinline__ float pair_factor(uint64_t seed, int64_t pair)
 }
 
 constexpr int kRedThreads = 256;
+constexpr int kEdgeList = 64 * 8;  // gradient entries a wave gathers per side: every corner of every lane
 constexpr int64_t kEdgeDirectBlocks = 4096;  // grid-stride blocks of the fused edge loss (partials per call)
 
 // block total of one double per thread, valid in thread 0, in a fixed order: a butterfly within each wave, then the
@@ -216,16 +217,17 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
     if constexpr (kGrad)
         if (P > 0) gscale = (float)((double)*grad_loss * weight / (double)P);
     double acc = 0.0;
-    for (I i = (I)blockIdx.x * (I)blockDim.x + (I)threadIdx.x; i < total; i += (I)gridDim.x * (I)blockDim.x)
-    {
+    // one lane's pair: its channels' loss terms into acc and their gradients into gv; false when the lane has no pair
+    auto eval = [&](I i, int64_t& sa, int64_t& so, TriLocal& ta, TriLocal& to, float (&gv)[4], int32_t& ch0) -> bool {
         const I c       = i / quads;
         const int32_t o = other[c];
-        if (o < 0) continue;
-        const int32_t ch0  = 4 * (int32_t)(i - c * quads);
+        if (o < 0) return false;
+        ch0                = 4 * (int32_t)(i - c * quads);
         const Candidate cd = split_candidate<I>(c, G);
         const int32_t node = (int32_t)active_ids[cd.aidx];
-        const int64_t sa = node_slot[node], so = node_slot[o];
-        if (sa < 0 || sa >= g.N || so < 0 || so >= g.N) continue;  // the grid sample reads zeros there
+        sa = node_slot[node];
+        so = node_slot[o];
+        if (sa < 0 || sa >= g.N || so < 0 || so >= g.N) return false;  // the grid sample reads zeros there
         float p[3];
         face_point(pmin, pmax, node, cd.side, cd.front, cd.sid, G, p);
         float ua[3], uo[3];
@@ -237,8 +239,8 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
             ua[d] = (p[d] - mna) / (mxa - mna) * 2 - 1;
             uo[d] = (p[d] - mno) / (mxo - mno) * 2 - 1;
         }
-        const TriLocal ta = trilinear_local(g, ua[0], ua[1], ua[2]);
-        const TriLocal to = trilinear_local(g, uo[0], uo[1], uo[2]);
+        ta = trilinear_local(g, ua[0], ua[1], ua[2]);
+        to = trilinear_local(g, uo[0], uo[1], uo[2]);
         const float* ga   = g.grid + sa * g.s0;
         const float* go   = g.grid + so * g.s0;
         float fa[4] = {0.f, 0.f, 0.f, 0.f}, fo[4] = {0.f, 0.f, 0.f, 0.f};
@@ -276,7 +278,6 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
         }
         const float r = pair_factor(seed, row[c]);
         const int nch = min(4, g.C - ch0);
-        float gv[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
         {
@@ -287,20 +288,87 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
             }
             gv[j] = j < nch ? gscale * r * sgn(d) : 0.f;
         }
-        if constexpr (kGrad)
+        return true;
+    };
+    const I stride = (I)gridDim.x * (I)blockDim.x;
+    if constexpr (kGrad && kVec4)
+    {
+        // The gradient's atomics, coalesced: the lanes of a wave append what they add (gradient quad, corner address,
+        // weight; corners of weight zero and quads of zero gradient add nothing) to a list in LDS, and the wave then
+        // takes 16 entries at a time, four lanes to the four consecutive channels of one. Issued from the pairs'
+        // lanes directly, each of an instruction's 64 adds is a request of its own.
+        // Measured on 4096 random grids of 17^3 x 8 (7.1 M candidates): 2.97 ms with the pairs' lanes adding
+        // directly, 1.04 ms like this (0.61 ms without any add).
+        __shared__ float4 s_gv[kRedThreads];
+        __shared__ int64_t s_off[kRedThreads / 64][kEdgeList];
+        __shared__ float2 s_w[kRedThreads / 64][kEdgeList];  // weight (signed), lane
+        __shared__ int32_t s_n[kRedThreads / 64];
+        const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+        // uniform trip count over the wave: every lane takes part in every list
+        for (I i0 = (I)blockIdx.x * (I)blockDim.x + (I)(threadIdx.x & ~63u); i0 < total; i0 += stride)
         {
-            float* da = grad_grid + sa * g.s0;
-            float* dq = grad_grid + so * g.s0;
+            const I i = i0 + (I)l;
+            int64_t sa = 0, so = 0;
+            TriLocal ta, to;
+            float gv[4] = {0.f, 0.f, 0.f, 0.f};
+            int32_t ch0 = 0;
+            const bool has = i < total && eval(i, sa, so, ta, to, gv, ch0) &&
+                             (gv[0] != 0.f || gv[1] != 0.f || gv[2] != 0.f || gv[3] != 0.f);
+            s_gv[threadIdx.x] = make_float4(gv[0], gv[1], gv[2], gv[3]);
+            for (int side = 0; side < 2; ++side)
+            {
+                if (l == 0) s_n[wave] = 0;
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                if (has)
+                {
+                    const TriLocal& t  = side ? to : ta;
+                    const int64_t base = (side ? so : sa) * g.s0 + ch0;
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (ta.w[k] != 0.f)
-                    for (int j = 0; j < nch; ++j)
-                        if (gv[j] != 0.f) atomicAdd(da + ta.off[k] + (ch0 + j) * (int32_t)g.s1, ta.w[k] * gv[j]);
+                    for (int k = 0; k < 8; ++k)
+                    {
+                        if (t.w[k] == 0.f) continue;
+                        const int32_t e = atomicAdd(&s_n[wave], 1);
+                        s_off[wave][e]  = base + t.off[k];
+                        s_w[wave][e]    = make_float2(side ? -t.w[k] : t.w[k], __int_as_float(threadIdx.x));
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                const int32_t n = s_n[wave];
+                for (int32_t e = l >> 2; e < n; e += 16)
+                {
+                    const float2 w = s_w[wave][e];
+                    const float v  = reinterpret_cast<const float*>(&s_gv[__float_as_int(w.y)])[l & 3];
+                    if (v != 0.f) atomicAdd(grad_grid + s_off[wave][e] + (l & 3), w.x * v);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            }
+        }
+    }
+    else
+    {
+        for (I i = (I)blockIdx.x * (I)blockDim.x + (I)threadIdx.x; i < total; i += stride)
+        {
+            int64_t sa, so;
+            TriLocal ta, to;
+            float gv[4];
+            int32_t ch0;
+            if (!eval(i, sa, so, ta, to, gv, ch0)) continue;
+            if constexpr (kGrad)
+            {
+                const int nch = min(4, g.C - ch0);
+                float* da = grad_grid + sa * g.s0;
+                float* dq = grad_grid + so * g.s0;
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (to.w[k] != 0.f)
-                    for (int j = 0; j < nch; ++j)
-                        if (gv[j] != 0.f) atomicAdd(dq + to.off[k] + (ch0 + j) * (int32_t)g.s1, to.w[k] * -gv[j]);
+                for (int k = 0; k < 8; ++k)
+                    if (ta.w[k] != 0.f)
+                        for (int j = 0; j < nch; ++j)
+                            if (gv[j] != 0.f) atomicAdd(da + ta.off[k] + (ch0 + j) * (int32_t)g.s1, ta.w[k] * gv[j]);
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    if (to.w[k] != 0.f)
+                        for (int j = 0; j < nch; ++j)
+                            if (gv[j] != 0.f) atomicAdd(dq + to.off[k] + (ch0 + j) * (int32_t)g.s1, to.w[k] * -gv[j]);
+            }
         }
     }
     if constexpr (kLoss) block_sum_to(acc, partials);
