@@ -2,15 +2,18 @@
 // forward and backward in FP32.
 //
 // The projector's decoder shape (8 inputs, one hidden layer of 32 or 64 relu or silu units, one output) runs on the
-// matrix cores (v_mfma_f32_32x32x2f32, the tiles of mfma_mlp.hpp): persistent workgroups of 4 waves, one tile of 32
-// samples per wave at a time, weights laid out once per workgroup in LDS. Other shapes run the vector-ALU tiles of
-// mlp_tile.hpp, one wave per tile of 64 samples.
+// matrix cores: persistent workgroups, one tile of 32 samples per wave at a time, weights laid out once per workgroup
+// in LDS. The forward and the relu backward take their products in split form on the BF16 matrix cores (split_mlp.hpp),
+// the silu backward on the FP32 ones (v_mfma_f32_32x32x2f32, the tiles of mfma_mlp.hpp). Other shapes run the
+// vector-ALU tiles of mlp_tile.hpp, one wave per tile of 64 samples. On 10^6 rows with H = 64, relu, forward and
+// backward took 112 and 484 us on the FP32 matrix cores and take 60 and 195 us in split form.
 //
-// Backward (both forms): each wave or workgroup recomputes its tiles' forward, back-propagates, and accumulates its
+// Backward (all forms): each wave or workgroup recomputes its tiles' forward, back-propagates, and accumulates its
 // share of the parameter gradient into its own slice of a partials buffer (every entry written by one thread); a
 // second kernel sums the slices in a fixed order, so the result is deterministic.
 #include "mfma_mlp.hpp"
 #include "mlp_tile.hpp"
+#include "split_mlp.hpp"
 
 namespace neat
 {
@@ -82,29 +85,62 @@ __device__ __forceinline__ void load_x4(const float* __restrict__ x, int64_t i, 
     for (int j = 0; j < 4; ++j) x4[j] = i < S ? x[i * 8 + 4 * hg + j] : 0.f;
 }
 
+// Forward: the products in split form on the BF16 matrix cores (split_mlp.hpp). Tiles go round the workgroups first, so
+// that a few rows spread over the CUs.
+constexpr int kDecFwdThreads = 768;  // 12 waves, three per SIMD
+
 template <int H, int ACT>
-__global__ void __launch_bounds__(256, 2) k_dec_mfma_fwd(const float* __restrict__ x, int64_t S,
-                                                      const float* __restrict__ params, int last_act, float beta,
-                                                      float* __restrict__ y)
+__global__ void __launch_bounds__(kDecFwdThreads, 3) k_dec_split_fwd(const float* __restrict__ x, int64_t S,
+                                                                     const float* __restrict__ params, int last_act,
+                                                                     float beta, float* __restrict__ y)
 {
-    typedef PrecF32 P;
-    __shared__ WeightLDS<P, H> w;
-    load_weights<P, H, 8>(params, w);
-    __syncthreads();
+    __shared__ WeightLDSSplitFwd<H> w;
+    load_weights_split_fwd<H>(params, w);
     const int l = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t tiles = (S + 31) / 32;
-    for (int64_t t = (int64_t)blockIdx.x * kDecMfmaWaves + wave; t < tiles; t += (int64_t)gridDim.x * kDecMfmaWaves)
+    for (int64_t t = blockIdx.x + (int64_t)gridDim.x * wave; t < tiles; t += (int64_t)gridDim.x * (kDecFwdThreads / 64))
     {
         const int64_t i = t * 32 + (l & 31);
         float x4[4];
         load_x4(x, i, S, x4);
-        Fwd<H / 32> f;
-        tile_forward_mfma<P, H, ACT>(w, x4, beta, f);
-        if (i < S && l < 32) y[i] = act_f(last_act, f.z, beta);
+        const float z = tile_forward_split<H, ACT>(params, w, x4, beta);
+        if (i < S && l < 32) y[i] = act_f(last_act, z, beta);
     }
 }
 
-// One partial slice per wave (kDecMfmaWaves per workgroup).
+// Backward for relu, in split form; one partial slice per workgroup.
+constexpr int kDecBwdThreads = 512;  // 8 waves, two per SIMD
+
+template <int H>
+__global__ void __launch_bounds__(kDecBwdThreads, 2) k_dec_split_bwd(const float* __restrict__ x, int64_t S,
+                                                                     const float* __restrict__ params, int last_act,
+                                                                     float beta, const float* __restrict__ gy,
+                                                                     float* __restrict__ gx,
+                                                                     float* __restrict__ partials, int32_t P_total)
+{
+    __shared__ WeightLDSSplit<H> w;
+    __shared__ __align__(16) SplitStage stage[kDecBwdThreads / 64];
+    load_weights_split<H>(params, w);
+    const int l = threadIdx.x & 63, wave = threadIdx.x >> 6, hg = l >> 5;
+    SplitAcc<H / 32> acc;
+    const int64_t tiles = (S + 31) / 32;
+    for (int64_t t = blockIdx.x + (int64_t)gridDim.x * wave; t < tiles; t += (int64_t)gridDim.x * (kDecBwdThreads / 64))
+    {
+        const int64_t i  = t * 32 + (l & 31);
+        const bool valid = i < S;
+        float x4[4], dx[4];
+        load_x4(x, i, S, x4);
+        tile_backward_split<H>(params, w, x4, valid ? gy[i] : 0.f, valid, last_act, beta, stage[wave], acc, dx);
+        if (gx && valid)
+        {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) gx[i * 8 + 4 * hg + j] = dx[j];
+        }
+    }
+    write_split_partials<H>(params, w, acc, stage, partials + (int64_t)blockIdx.x * P_total);
+}
+
+// Backward for silu on the FP32 matrix cores; one partial slice per wave (kDecMfmaWaves per workgroup).
 template <int H, int ACT>
 __global__ void __launch_bounds__(256) k_dec_mfma_bwd(const float* __restrict__ x, int64_t S,
                                                       const float* __restrict__ params, int last_act, float beta,
@@ -204,18 +240,15 @@ extern "C"
         hipStream_t s = as_stream(stream);
         if (dec_mfma(in, hidden, layers, out, act))
         {
-            const int64_t tiles = (S + 31) / 32;
-            const unsigned wg =
-                (unsigned)std::max<int64_t>(1, std::min<int64_t>((tiles + kDecMfmaWaves - 1) / kDecMfmaWaves,
-                                                                 (int64_t)device_cus() * 8));
+            const unsigned wg = (unsigned)std::min<int64_t>((S + 31) / 32, device_cus());
             if (hidden == 32 && act == NEAT_ACT_RELU)
-                k_dec_mfma_fwd<32, NEAT_ACT_RELU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, y);
+                k_dec_split_fwd<32, NEAT_ACT_RELU><<<wg, kDecFwdThreads, 0, s>>>(x, S, params, last_act, beta, y);
             else if (hidden == 32)
-                k_dec_mfma_fwd<32, NEAT_ACT_SILU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, y);
+                k_dec_split_fwd<32, NEAT_ACT_SILU><<<wg, kDecFwdThreads, 0, s>>>(x, S, params, last_act, beta, y);
             else if (act == NEAT_ACT_RELU)
-                k_dec_mfma_fwd<64, NEAT_ACT_RELU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, y);
+                k_dec_split_fwd<64, NEAT_ACT_RELU><<<wg, kDecFwdThreads, 0, s>>>(x, S, params, last_act, beta, y);
             else
-                k_dec_mfma_fwd<64, NEAT_ACT_SILU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, y);
+                k_dec_split_fwd<64, NEAT_ACT_SILU><<<wg, kDecFwdThreads, 0, s>>>(x, S, params, last_act, beta, y);
             NEAT_LAUNCHED();
             return NEAT_OK;
         }
@@ -255,18 +288,23 @@ extern "C"
         float* partials = wt + P;
         if (dec_mfma(in, hidden, layers, out, act))
         {
-            // kDecMfmaWaves slices per workgroup, within the bwd_workgroups(S) slices the workspace holds
-            const int wg = std::max(1, std::min(bwd_workgroups(S) / kDecMfmaWaves, device_cus()));
+            // one slice per workgroup (relu) or kDecMfmaWaves, within the bwd_workgroups(S) slices the workspace holds
+            int wg = std::min(bwd_workgroups(S), device_cus()), slices = wg;
+            if (act != NEAT_ACT_RELU)
+            {
+                wg     = std::max(1, std::min(bwd_workgroups(S) / kDecMfmaWaves, device_cus()));
+                slices = wg * kDecMfmaWaves;
+            }
             if (hidden == 32 && act == NEAT_ACT_RELU)
-                k_dec_mfma_bwd<32, NEAT_ACT_RELU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
+                k_dec_split_bwd<32><<<wg, kDecBwdThreads, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
+            else if (act == NEAT_ACT_RELU)
+                k_dec_split_bwd<64><<<wg, kDecBwdThreads, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
             else if (hidden == 32)
                 k_dec_mfma_bwd<32, NEAT_ACT_SILU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
-            else if (act == NEAT_ACT_RELU)
-                k_dec_mfma_bwd<64, NEAT_ACT_RELU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
             else
                 k_dec_mfma_bwd<64, NEAT_ACT_SILU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
             NEAT_LAUNCHED();
-            k_dec_reduce_partials<<<reduce_partials_blocks(P), 256, 0, s>>>(partials, wg * kDecMfmaWaves, P, gparams);
+            k_dec_reduce_partials<<<reduce_partials_blocks(P), 256, 0, s>>>(partials, slices, P, gparams);
             NEAT_LAUNCHED();
             return NEAT_OK;
         }

@@ -214,9 +214,8 @@ __device__ __forceinline__ typename P::Frag1 x_step(const float (&x4)[4], int s)
     }
 }
 
-template <typename P, int H, int ACT>
-__device__ __forceinline__ void tile_forward_mfma(const WeightLDS<P, H>& w, const float (&x4)[4], float beta,
-                                                  Fwd<H / 32>& f)
+template <typename P, int H, int ACT, typename WS>
+__device__ __forceinline__ void tile_forward_mfma(const WS& w, const float (&x4)[4], float beta, Fwd<H / 32>& f)
 {
     constexpr int MT = H / 32, S = steps_per_tile<P>();
     const int l = threadIdx.x & 63, g = l >> 5;
@@ -510,6 +509,46 @@ __device__ __forceinline__ void write_param_partials(BwdAcc<H / 32>& acc, float*
 #pragma unroll
     for (int off = 16; off >= 1; off >>= 1) b3 += __shfl_xor(b3, off);
     if (l == 0) part[ob2] = b3;
+}
+
+// ---- fragment transposes through LDS ------------------------------------------------------------------------------
+// An "h" fragment (samples on the lanes: lane (n, g) holds rows 16st + 8(j/4) + 4g + j%4 of sample n for slot j) and
+// the "s" fragment of the same 32 x 32 tile (lane (m, g) holds samples crow(8st + j, g) of row m) are transposes of
+// each other. The h fragments of a tile go to a per-wave LDS tile [sample][row] (rows padded to 36 elements, 72 B,
+// so consecutive samples start on different banks) with two 8-byte stores each; the s fragments come back with
+// ds_read_b64_tr_b16, which hands lane 16G + i of a 16-lane group element e of the 8 bytes that lane 16G + 4e + i/4
+// points at, shifted by i % 4 elements: with lane 16G + 4e + q pointing at (sample 16st + 8r + 4(G/2) + e,
+// row 16(G%2) + 4q), lane (m, g) receives rows m of samples 16st + 8r + 4g + e, the s-fragment slots 4r + e.
+constexpr int kTrRow = 36;  // bf16 elements per sample row of a transpose tile
+
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+#define NEAT_LDS __attribute__((address_space(3)))
+
+__device__ __forceinline__ void tr_store(unsigned short* tile, const bf16x8& f, int st)
+{
+    const int l = threadIdx.x & 63, n = l & 31, g = l >> 5;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 v = __builtin_bit_cast(u32x4, f);
+    unsigned short* row = tile + n * kTrRow + 16 * st + 4 * g;
+    *reinterpret_cast<uint2*>(row)     = make_uint2(v[0], v[1]);
+    *reinterpret_cast<uint2*>(row + 8) = make_uint2(v[2], v[3]);
+}
+
+__device__ __forceinline__ bf16x8 tr_load(const unsigned short* tile, int st)
+{
+    const int l = threadIdx.x & 63, G = l >> 4, e = (l >> 2) & 3, q = l & 3;
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    u32x2 r[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+    {
+        const unsigned short* src = tile + (16 * st + 8 * h + 4 * (G >> 1) + e) * kTrRow + 16 * (G & 1) + 4 * q;
+        const s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((NEAT_LDS s16x4_t*)(src));
+        r[h]            = __builtin_bit_cast(u32x2, v);
+    }
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 o = {r[0][0], r[0][1], r[1][0], r[1][1]};
+    return __builtin_bit_cast(bf16x8, o);
 }
 
 // ---- BF16 relu decoders: weights for products in both orientations --------------------------------------------

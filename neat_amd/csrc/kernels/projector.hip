@@ -737,12 +737,14 @@ __global__ void __launch_bounds__(256) k_fill_f32(float* p, int64_t n, float v)
     if (i < n) p[i] = v;
 }
 
-// Forward: persistent workgroups of 4 waves over the chunks; tiles of 32 samples per wave on the matrix cores;
-// per-segment sums sequential in j as in k_proj_fwd.
-template <typename P, int H, int ACT>
+// Forward of the BF16 form where the node-resident relu kernel does not apply (silu, or a node grid over 17^3):
+// persistent workgroups of 4 waves over the chunks; tiles of 32 samples per wave on the matrix cores; per-segment
+// sums sequential in j as in k_proj_fwd.
+template <int H, int ACT>
 __global__ void __launch_bounds__(256, 2) k_mfma_fwd(ProjGeom g, Plan p, const float* __restrict__ params,
                                                   const void* grid_lowp, float* seg_partial, float* sample_out)
 {
+    typedef PrecBF16 P;
     __shared__ WeightLDS<P, H> w;
     __shared__ ChunkCtx cx;
     __shared__ float s_contrib[kFwdChunk];
@@ -975,6 +977,8 @@ int node_workgroups()
 int bw1_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::min<int64_t>(z.max1, 2048)); }
 // matrix-core backward: persistent workgroups of 4 waves, one partial slice per wave
 int mfma_bwd_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::min<int64_t>(z.max1, 256)); }
+// split forward: persistent workgroups, one per CU (their LDS)
+int split_fwd_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::min<int64_t>(z.max1, 256)); }
 int mfma_fwd_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::min<int64_t>(z.max1, 1024)); }
 
 size_t partials_bytes(const ProjSizes& z)
@@ -1131,18 +1135,27 @@ int launch_fwd_valu(hipStream_t s, const Args& a, const Plan& p, float* seg_part
 template <typename P, int H>
 int launch_fwd_mfma(hipStream_t s, const Args& a, const Plan& p, float* seg_partial, float* sample_out = nullptr)
 {
-    const unsigned grid = (unsigned)mfma_fwd_workgroups(a.z);
-    if (P::kBF16 && a.relu16)
+    if constexpr (!P::kBF16)
     {
-        NEAT_REQUIRE(launch_mfma_fwd_relu(s, H, a.g, p, a.params, a.grid_bf16, seg_partial, sample_out) == 0,
-                     "k_mfma_fwd_relu launch failed");
-        return NEAT_OK;
+        NEAT_REQUIRE(launch_split_fwd(s, H, a.act, split_fwd_workgroups(a.z), a.g, p, a.params, seg_partial,
+                                      sample_out) == 0,
+                     "k_split_fwd launch failed");
     }
-    if (a.act == NEAT_ACT_RELU)
-        k_mfma_fwd<P, H, NEAT_ACT_RELU><<<grid, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, seg_partial, sample_out);
     else
-        k_mfma_fwd<P, H, NEAT_ACT_SILU><<<grid, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, seg_partial, sample_out);
-    NEAT_LAUNCHED();
+    {
+        const unsigned grid = (unsigned)mfma_fwd_workgroups(a.z);
+        if (a.relu16)
+        {
+            NEAT_REQUIRE(launch_mfma_fwd_relu(s, H, a.g, p, a.params, a.grid_bf16, seg_partial, sample_out) == 0,
+                         "k_mfma_fwd_relu launch failed");
+            return NEAT_OK;
+        }
+        if (a.act == NEAT_ACT_RELU)
+            k_mfma_fwd<H, NEAT_ACT_RELU><<<grid, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, seg_partial, sample_out);
+        else
+            k_mfma_fwd<H, NEAT_ACT_SILU><<<grid, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, seg_partial, sample_out);
+        NEAT_LAUNCHED();
+    }
     return NEAT_OK;
 }
 
@@ -1219,7 +1232,10 @@ int launch_bw_mfma(hipStream_t s, const Args& a, const Plan& p, const BwdBufs& b
 {
     // BF16 with relu hidden layers runs k_mfma_bwd_relu (node-resident: p.nwg workgroups of kNodeWaves waves)
     const bool relu16 = P::kBF16 && a.relu16;
-    const int slices  = relu16 ? p.nwg * kNodeWaves : mfma_bwd_workgroups(a.z) * 4;
+    // FP32 with relu hidden layers runs k_split_bwd (the masks it folds into its products need relu)
+    const bool relu32 = !P::kBF16 && a.act == NEAT_ACT_RELU;
+    const int nwg     = mfma_bwd_workgroups(a.z);
+    const int slices  = relu16 ? p.nwg * kNodeWaves : (relu32 ? nwg : nwg * 4);
     const int Ptot    = a.m.nparams();
     if (stage == 1)
     {
@@ -1232,13 +1248,27 @@ int launch_bw_mfma(hipStream_t s, const Args& a, const Plan& p, const BwdBufs& b
             NEAT_REQUIRE(rc == 0, "k_mfma_bwd_relu launch failed");
             return NEAT_OK;
         }
-        const int nwg = mfma_bwd_workgroups(a.z);
-        if (a.act == NEAT_ACT_RELU)
-            k_mfma_bwd<P, H, NEAT_ACT_RELU><<<nwg, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, b.grad_proj, b.dfeat,
-                                                                 b.sgc, b.dmax, b.partials, Ptot);
+        if constexpr (P::kBF16)
+        {
+            if (a.act == NEAT_ACT_RELU)
+                k_mfma_bwd<P, H, NEAT_ACT_RELU><<<nwg, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, b.grad_proj,
+                                                                     b.dfeat, b.sgc, b.dmax, b.partials, Ptot);
+            else
+                k_mfma_bwd<P, H, NEAT_ACT_SILU><<<nwg, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, b.grad_proj,
+                                                                     b.dfeat, b.sgc, b.dmax, b.partials, Ptot);
+        }
         else
+        {
+            if (relu32)
+            {
+                const int rc = launch_split_bwd(s, H, nwg, a.g, p, a.params, b.grad_proj, b.dfeat, b.sgc, b.dmax,
+                                                b.partials, Ptot);
+                NEAT_REQUIRE(rc == 0, "k_split_bwd launch failed");
+                return NEAT_OK;
+            }
             k_mfma_bwd<P, H, NEAT_ACT_SILU><<<nwg, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, b.grad_proj, b.dfeat,
                                                                  b.sgc, b.dmax, b.partials, Ptot);
+        }
         NEAT_LAUNCHED();
         return NEAT_OK;
     }

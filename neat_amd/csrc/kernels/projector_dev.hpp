@@ -659,4 +659,14 @@ int launch_mfma_fwd_relu(hipStream_t s, int H, const ProjGeom& g, const Plan& p,
 int launch_mfma_bwd_relu(hipStream_t s, int H, const ProjGeom& g, const Plan& p, const float* params,
                          const float* grad_proj, float* dfeat, unsigned int* dmax, float* partials, int32_t P_total);
 
+// ---- FP32 forward and relu backward in split form (projector_fp32.hip) --------------------------------------------
+int launch_split_fwd(hipStream_t s, int H, int act, int workgroups, const ProjGeom& g, const Plan& p,
+                     const float* params, float* seg_partial, float* sample_out);
+
+// Launches k_split_bwd<H> (H = 32 or 64): writes dL/dfeature and the grid coordinates of every sample, the batch's
+// largest |dL/dfeature|, and one parameter-gradient slice per workgroup.
+int launch_split_bwd(hipStream_t s, int H, int workgroups, const ProjGeom& g, const Plan& p, const float* params,
+                     const float* grad_proj, float* dfeat, float4* sgc, unsigned int* dmax, float* partials,
+                     int32_t P_total);
+
 }  // namespace neat
