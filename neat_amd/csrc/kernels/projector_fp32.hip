@@ -3,7 +3,7 @@
 //
 // On the FP32 matrix cores a tile of 32 samples with H = 64 took 4,608 cycles of products forward and 21,000 backward
 // (a 32x32x2 product is 64 cycles); in split form it is 1,730 and 4,160, beside about 2,200 and 5,900 cycles of vector
-// work. Measured on 53.3 M samples (2^18 rays, 4096 grids of 17^3 x 8): forward 7.37 -> 3.5 ms, backward 28.3 -> 9.2 ms
+// work. Measured on 53.3 M samples (2^18 rays, 4096 grids of 17^3 x 8): forward 7.37 -> 3.5 ms, backward 28.3 -> 8.3 ms
 // (10.9 with every pre-activation recomputed on the FP32 matrix cores; 0.5 ms are the tiles that are). The gather of
 // the node grid takes about 1.3 ms of the backward; two waves per SIMD leave the matrix cores idle two thirds of the
 // time, the rest being vector work and exposed LDS latency.
@@ -30,8 +30,8 @@ __global__ void __launch_bounds__(kSplitThreads, 2) k_split_bwd(ProjGeom g, Plan
     SplitStage& sg = stage[wave];
     SplitAcc<H / 32> acc;
     float amax = 0.f;  // largest |dL/dfeature| this lane wrote
-    const int64_t nchunks = p.chunk_off1[g.N];
-    for (int64_t c = blockIdx.x; c < nchunks; c += gridDim.x)
+    const int32_t nchunks = (int32_t)p.chunk_off1[g.N];
+    for (int32_t c = blockIdx.x; c < nchunks; c += (int32_t)gridDim.x)
     {
         const int32_t slot = p.chunk1_slot[c];
         const int32_t q0 = p.chunk1_q0[c], q1 = p.chunk1_q1[c], nseg = q1 - q0;
@@ -97,8 +97,8 @@ __global__ void __launch_bounds__(kSplitFwdThreads, 3) k_split_fwd(ProjGeom g, P
     __shared__ float s_seg[kSegCap];
     load_weights_split_fwd<H>(params, w);
     const int l = threadIdx.x & 63, wave = threadIdx.x >> 6, n = l & 31, hg = l >> 5;
-    const int64_t nchunks = p.chunk_off1[g.N];
-    for (int64_t c = blockIdx.x; c < nchunks; c += gridDim.x)
+    const int32_t nchunks = (int32_t)p.chunk_off1[g.N];
+    for (int32_t c = blockIdx.x; c < nchunks; c += (int32_t)gridDim.x)
     {
         const int32_t slot = p.chunk1_slot[c];
         const int32_t q0 = p.chunk1_q0[c], q1 = p.chunk1_q1[c], nseg = q1 - q0;
