@@ -329,40 +329,52 @@ __device__ __forceinline__ int32_t find_segment(const int64_t* nm_soff, int32_t 
 }
 
 // ---- matrix-core path ---------------------------------------------------------------------------------------------------
-// Gather of the lane's 4 channels (group g: channels 4g..4g+3) of an 8-channel node grid, FP32 or BF16 storage,
-// trilinear weights and accumulation in FP32 (same corner order as the reference).
+// The lane's 4 channels (group g: channels 4g..4g+3) of corner vertex `off` of an 8-channel node grid, FP32 or BF16.
 template <bool kBF16Grid>
-__device__ __forceinline__ void gather_half(const void* node_grid, const Corners& c, int g, float (&x4)[4])
+struct CornerRaw
+{
+    typedef typename std::conditional<kBF16Grid, uint2, float4>::type T;
+    __device__ static __forceinline__ T load(const void* node_grid, int off, int g)
+    {
+        if constexpr (kBF16Grid)
+            return *reinterpret_cast<const uint2*>(static_cast<const unsigned short*>(node_grid) + off + 4 * g);
+        else
+            return *reinterpret_cast<const float4*>(static_cast<const float*>(node_grid) + off + 4 * g);
+    }
+    __device__ static __forceinline__ float4 value(const T& raw)
+    {
+        if constexpr (kBF16Grid)
+            return make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u),
+                               __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xFFFF0000u));
+        else
+            return raw;
+    }
+};
+
+// Trilinear sum of the 8 corners, weights and accumulation in FP32 (same corner order as the reference).
+template <bool kBF16Grid>
+__device__ __forceinline__ void gather_sum(const typename CornerRaw<kBF16Grid>::T (&raw)[8], const float (&w)[8],
+                                           float (&x4)[4])
 {
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int k = 0; k < 8; ++k)
     {
-        float4 v;
-        if constexpr (kBF16Grid)
-        {
-            uint2 raw = *reinterpret_cast<const uint2*>(static_cast<const unsigned short*>(node_grid) + c.off[k] + 4 * g);
-            v = make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u),
-                            __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xFFFF0000u));
-        }
-        else
-        {
-            v = *reinterpret_cast<const float4*>(static_cast<const float*>(node_grid) + c.off[k] + 4 * g);
-        }
+        const float4 v = CornerRaw<kBF16Grid>::value(raw[k]);
         if constexpr (kBF16Grid)
         {
             // the BF16 form is not bound to the oracle's rounding: fused multiply-adds
-            acc.x = fmaf(v.x, c.w[k], acc.x);
-            acc.y = fmaf(v.y, c.w[k], acc.y);
-            acc.z = fmaf(v.z, c.w[k], acc.z);
-            acc.w = fmaf(v.w, c.w[k], acc.w);
+            acc.x = fmaf(v.x, w[k], acc.x);
+            acc.y = fmaf(v.y, w[k], acc.y);
+            acc.z = fmaf(v.z, w[k], acc.z);
+            acc.w = fmaf(v.w, w[k], acc.w);
         }
         else
         {
-            acc.x += v.x * c.w[k];
-            acc.y += v.y * c.w[k];
-            acc.z += v.z * c.w[k];
-            acc.w += v.w * c.w[k];
+            acc.x += v.x * w[k];
+            acc.y += v.y * w[k];
+            acc.z += v.z * w[k];
+            acc.w += v.w * w[k];
         }
     }
     x4[0] = acc.x;
@@ -567,7 +579,7 @@ __device__ __forceinline__ void node_bounds(const ProjGeom& g, int32_t node, Nod
 // sample p0 + n (tile A) and p0 + 32 + n (tile B) and gathers its 4 channels of both. v is the sample weight
 // (forward) or dL/dy = dL/dproj x weight (backward); samples past the window have zero weights, features and v.
 // The backward also stores each sample's grid coordinate for the scatter: (ix, iy, iz, 0) in the FP32 form, the
-// packed cell and fractions (pack_cell_coord) in the BF16 form. A BF16 forward given sgc and w_out stores the packed
+// packed cell and fractions (pack_cell_coord) in the BF16 form. kGlobal: the grid is in global memory (not in LDS). A BF16 forward given sgc and w_out stores the packed
 // coordinate and the sample weight (what its backward reads instead of recomputing them).
 struct PairIn
 {
@@ -575,7 +587,7 @@ struct PairIn
     float va, vb;
 };
 
-template <bool kBF16, bool kBwd>
+template <bool kBF16, bool kBwd, bool kGlobal = true>
 __device__ __forceinline__ void fetch_pair(const ProjGeom& g, const ChunkCtx& cx, int32_t p0, int32_t w0,
                                            int32_t wn, int64_t base, const NodeBox& nb, const void* ngrid,
                                            float4* sgc, PairIn& in, float* w_out = nullptr)
@@ -624,8 +636,17 @@ __device__ __forceinline__ void fetch_pair(const ProjGeom& g, const ChunkCtx& cx
         cb.w[k]      = __uint_as_float(w[1]);
     }
     const auto vv = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    gather_half<kBF16>(ngrid, ca, hg, in.xa);
-    gather_half<kBF16>(ngrid, cb, hg, in.xb);
+    // every load of the pair is issued before the first sum: left to itself the compiler, short of registers in the
+    // backward, waits for one corner after the other
+    typedef CornerRaw<kBF16> CR;
+    typename CR::T ra[8], rb[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) ra[k] = CR::load(ngrid, ca.off[k], hg);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) rb[k] = CR::load(ngrid, cb.off[k], hg);
+    if constexpr (kGlobal) __builtin_amdgcn_sched_barrier(0);
+    gather_sum<kBF16>(ra, ca.w, in.xa);
+    gather_sum<kBF16>(rb, cb.w, in.xb);
     in.va = __uint_as_float(vv[0]);
     in.vb = __uint_as_float(vv[1]);
 }

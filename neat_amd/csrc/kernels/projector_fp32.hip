@@ -25,7 +25,7 @@ __global__ void __launch_bounds__(kSplitThreads, 2) k_split_bwd(ProjGeom g, Plan
     __shared__ WeightLDSSplit<H> w;
     __shared__ ChunkCtx cx;
     __shared__ __align__(16) SplitStage stage[kSplitThreads / 64];
-    load_weights_split<H>(params, w);
+    load_weights_split<H>(params, reinterpret_cast<float*>(&stage[0]), w);
     const int l = threadIdx.x & 63, wave = threadIdx.x >> 6, hg = l >> 5;
     SplitStage& sg = stage[wave];
     SplitAcc<H / 32> acc;

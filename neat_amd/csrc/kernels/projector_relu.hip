@@ -460,7 +460,7 @@ __global__ void __launch_bounds__(kNodeThreads, 2) k_mfma_fwd_relu(ProjGeom g, P
             {
                 // the fetch also leaves each sample's packed cell coordinate and weight for the backward
                 PairIn cur;
-                fetch_pair<true, false>(g, cx, p0, w0, wn, base, nb, s_grid, reinterpret_cast<float4*>(p.cell_cache),
+                fetch_pair<true, false, false>(g, cx, p0, w0, wn, base, nb, s_grid, reinterpret_cast<float4*>(p.cell_cache),
                                         cur, p.w_cache);
                 if (p.feat_cache)
                 {

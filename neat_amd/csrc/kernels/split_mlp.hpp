@@ -81,7 +81,7 @@ struct WeightLDSSplitFwd
 
 // Packed parameter layout as load_weights (C = 8). Ends in a barrier.
 template <int H>
-__device__ void load_weights_split_fwd(const float* __restrict__ params, WeightLDSSplitFwd<H>& w)
+__device__ void load_weights_split_fwd(const float* params, WeightLDSSplitFwd<H>& w)
 {
     constexpr int MT = H / 32, C = 8;
     const float* W0 = params;
@@ -334,15 +334,18 @@ struct WeightLDSSplit : WeightLDSSplitFwd<H>
     bf16x8 w1t[MT][2][64];
 };
 
-// Ends in a barrier.
+// `copy` (LDS, the parameters' size) takes the parameters first, in one pass over global memory: the layouts below read
+// them in scattered order, several passes. Ends in a barrier.
 template <int H>
-__device__ void load_weights_split(const float* __restrict__ params, WeightLDSSplit<H>& w)
+__device__ void load_weights_split(const float* __restrict__ params, float* copy, WeightLDSSplit<H>& w)
 {
     constexpr int MT = H / 32, C = 8;
-    const float* W0 = params;
+    for (int t = threadIdx.x; t < H * C + H + H * H + H + H + 1; t += blockDim.x) copy[t] = params[t];
+    __syncthreads();
+    const float* W0 = copy;
     const float* W1 = W0 + H * C + H;
     const float* W2 = W1 + H * H + H;
-    load_weights_split_fwd<H>(params, w);
+    load_weights_split_fwd<H>(copy, w);
     for (int t = threadIdx.x; t < MT * MT * 2 * 64; t += blockDim.x)
     {
         const int l = t % 64, st = (t / 64) % 2, ms = (t / 128) % MT, mt = t / (128 * MT);
@@ -607,14 +610,19 @@ __device__ __forceinline__ void tile_backward_split(const float* __restrict__ pa
     }
 }
 
-// A wave's sums written to `red` (add: added to it) in the packed parameter layout, the hidden layer's without the
-// row factor w3, the output weights' not at all.
+// Floats of a wave's sums as put_split_sums lays them out: G [H][H], E [H][32], b3.
+template <int H>
+constexpr int split_sums()
+{
+    return H * H + 32 * H + 1;
+}
+
+// A wave's sums written to `red` (add: added to it).
 template <int H>
 __device__ __forceinline__ void put_split_sums(SplitAcc<H / 32>& acc, float* red, bool add)
 {
-    constexpr int MT = H / 32, C = 8;
+    constexpr int MT = H / 32;
     const int l = threadIdx.x & 63, n = l & 31, hg = l >> 5;
-    const int oW0 = 0, ob0 = H * C, oW1 = ob0 + H, ob1 = oW1 + H * H, oW2 = ob1 + H, ob2 = oW2 + H;
     auto put = [&](int i, float v) { red[i] = add ? red[i] + v : v; };
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -622,65 +630,70 @@ __device__ __forceinline__ void put_split_sums(SplitAcc<H / 32>& acc, float* red
 #pragma unroll
         for (int i = 0; i < 16; ++i)
         {
-            const int r    = 32 * mt + crow(i, hg);
-            const float e  = acc.E[mt][i];
-            const float e1 = __shfl(e, l + 8), e2 = __shfl(e, l + 16), c1 = __shfl(e, l + 1), c2 = __shfl(e, l + 2);
-            if (n < C) put(oW0 + r * C + n, e + (e1 + e2));
-            if (n == kTOnes) put(ob0 + r, e);
-            if (n == kTDz) put(ob1 + r, e + (c1 + c2));
+            const int r = 32 * mt + crow(i, hg);
 #pragma unroll
-            for (int m1 = 0; m1 < MT; ++m1) put(oW1 + r * H + 32 * m1 + n, acc.G[mt][m1][i]);
+            for (int m1 = 0; m1 < MT; ++m1) put(r * H + 32 * m1 + n, acc.G[mt][m1][i]);
+            put(H * H + r * 32 + n, acc.E[mt][i]);
         }
     }
     float b3 = acc.b3;
 #pragma unroll
     for (int off = 16; off >= 1; off >>= 1) b3 += __shfl_xor(b3, off);
-    if (l == 0) put(ob2, b3);
+    if (l == 0) put(H * H + 32 * H, b3);
 }
 
-// The workgroup's parameter-gradient slice: its waves' sums added in a fixed order in LDS (in the transpose tiles, which
-// are done with; as many waves at a time as have room there), the output weights' gradient from them (SplitAcc), then
-// stored. NW waves; called by every thread.
+// The workgroup's parameter-gradient slice, in the packed layout: its waves' sums added in a fixed order in LDS (in the
+// transpose tiles, which are done with; as many waves at a time as have room there), the hidden layer's rows times
+// w3, the output weights' gradient from them (SplitAcc), then stored. NW waves; called by every thread.
 template <int H, int NW>
 __device__ __forceinline__ void write_split_partials(const float* __restrict__ params, const WeightLDSSplit<H>& w,
                                                      SplitAcc<H / 32>& acc, SplitStage (&stage)[NW], float* part)
 {
-    constexpr int oW1 = H * 8 + H, ob1 = oW1 + H * H, oW2 = ob1 + H, P = oW2 + H + 1;
-    constexpr int kFit = (int)(sizeof(stage) / (P * sizeof(float))), NS = kFit < NW ? kFit : NW;
-    static_assert(NS >= 1, "a slice fits the transpose tiles");
+    constexpr int C = 8, ob0 = H * C, oW1 = ob0 + H, ob1 = oW1 + H * H, oW2 = ob1 + H, ob2 = oW2 + H;
+    constexpr int Q = split_sums<H>(), kFit = (int)(sizeof(stage) / (Q * sizeof(float))), NS = kFit < NW ? kFit : NW;
+    static_assert(NS >= 1, "a wave's sums fit the transpose tiles");
     float* red = reinterpret_cast<float*>(&stage[0]);
     const int wave = threadIdx.x >> 6;
     __syncthreads();
     for (int k = 0; k < NW; k += NS)
     {
-        if (wave >= k && wave < k + NS) put_split_sums<H>(acc, red + (wave - k) * P, k > 0);
+        if (wave >= k && wave < k + NS) put_split_sums<H>(acc, red + (wave - k) * Q, k > 0);
         __syncthreads();
     }
-    for (int t = threadIdx.x; t < P; t += blockDim.x)
+    for (int t = threadIdx.x; t < Q; t += blockDim.x)
     {
         float v = red[t];
 #pragma unroll
-        for (int k = 1; k < NS; ++k) v += red[k * P + t];
+        for (int k = 1; k < NS; ++k) v += red[k * Q + t];
         red[t] = v;
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < P; t += blockDim.x)
+    const float* E = red + H * H;
+    for (int t = threadIdx.x; t < H * C; t += blockDim.x)
     {
-        if (t >= oW2 && t < oW2 + H) continue;
-        float v = red[t];
-        if (t >= oW1 && t < oW2) v *= w.vec[2][t < ob1 ? (t - oW1) / H : t - ob1];
-        part[t] = v;
+        const float* e = E + (t / C) * 32 + t % C;
+        part[t]        = e[0] + (e[8] + e[16]);
     }
+    for (int t = threadIdx.x; t < H * H; t += blockDim.x) part[oW1 + t] = red[t] * w.vec[2][t / H];
+    // 8 lanes to a row
     for (int t = threadIdx.x; t < 8 * H; t += blockDim.x)
     {
-        const int r = t >> 3, q = t & 7;
-        float v     = q == 0 ? w.vec[1][r] * red[ob1 + r] : 0.f;
+        const int r    = t >> 3, q = t & 7;
+        const float* e = E + r * 32 + kTDz;
+        const float gb = e[0] + (e[1] + e[2]);
+        float v        = q == 0 ? w.vec[1][r] * gb : 0.f;
 #pragma unroll
-        for (int c = 0; c < H; c += 8) v = fmaf(params[oW1 + r * H + c + q], red[oW1 + r * H + c + q], v);
+        for (int c = 0; c < H; c += 8) v = fmaf(params[oW1 + r * H + c + q], red[r * H + c + q], v);
 #pragma unroll
         for (int off = 4; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-        if (q == 0) part[oW2 + r] = v;
+        if (q == 0)
+        {
+            part[ob0 + r] = E[r * 32 + kTOnes];
+            part[ob1 + r] = gb * w.vec[2][r];
+            part[oW2 + r] = v;
+        }
     }
+    if (threadIdx.x == 0) part[ob2] = E[32 * H];
 }
 
 }  // namespace neat
