@@ -737,82 +737,16 @@ __global__ void __launch_bounds__(256) k_fill_f32(float* p, int64_t n, float v)
     if (i < n) p[i] = v;
 }
 
-// Forward of the BF16 form where the node-resident relu kernel does not apply (silu, or a node grid over 17^3):
-// persistent workgroups of 4 waves over the chunks; tiles of 32 samples per wave on the matrix cores; per-segment
-// sums sequential in j as in k_proj_fwd.
-template <int H, int ACT>
-__global__ void __launch_bounds__(256, 2) k_mfma_fwd(ProjGeom g, Plan p, const float* __restrict__ params,
-                                                  const void* grid_lowp, float* seg_partial, float* sample_out)
-{
-    typedef PrecBF16 P;
-    __shared__ WeightLDS<P, H> w;
-    __shared__ ChunkCtx cx;
-    __shared__ float s_contrib[kFwdChunk];
-    __shared__ float s_seg[kSegCap];
-    load_weights<P, H, 8>(params, w);
-    const int l = threadIdx.x & 63, wave = threadIdx.x >> 6, n = l & 31, hg = l >> 5;
-    const int64_t nchunks = p.chunk_off1[g.N];
-    for (int64_t c = blockIdx.x; c < nchunks; c += gridDim.x)
-    {
-        const int32_t slot = p.chunk1_slot[c];
-        const int32_t q0 = p.chunk1_q0[c], q1 = p.chunk1_q1[c], nseg = q1 - q0;
-        if (nseg == 0) continue;
-        const int64_t base = p.nm_soff[q0];
-        __syncthreads();  // the previous chunk's readers of cx / s_seg are done
-        load_chunk_ctx(g, p, q0, q1, base, nullptr, cx);
-        for (int32_t t = threadIdx.x; t < nseg; t += blockDim.x) s_seg[t] = 0.f;
-        NodeBox nb;
-        node_bounds(g, g.seg_node[p.perm[q0]], nb);
-        const void* ngrid = node_grid_ptr(g, grid_lowp, P::kBF16, slot);
-        __syncthreads();
-        const int32_t nsamp = cx.beg[nseg];
-        for (int32_t w0 = 0; w0 < nsamp; w0 += kFwdChunk)
-        {
-            const int32_t wn = min(kFwdChunk, nsamp - w0);
-            expand_window(cx, nseg, w0, wn);
-            __syncthreads();
-            // pairs of tiles per wave (fetch_pair)
-            auto tile = [&](int32_t i, const float (&x4)[4], float wgt) {
-                Fwd<H / 32> f;
-                tile_forward_mfma<P, H, ACT>(w, x4, g.beta, f);
-                if (i < wn && hg == 0)
-                {
-                    const float y = act_f(NEAT_ACT_SOFTPLUS, f.z, g.beta);
-                    s_contrib[i]  = y * wgt;
-                    if (sample_out) sample_out[base + w0 + i] = y;
-                }
-            };
-            for (int32_t p0 = wave * 64; p0 < wn; p0 += 256)
-            {
-                PairIn cur;
-                fetch_pair<P::kBF16, false>(g, cx, p0, w0, wn, base, nb, ngrid, nullptr, cur);
-                tile(p0 + n, cur.xa, cur.va);
-                if (p0 + 32 < wn) tile(p0 + 32 + n, cur.xb, cur.vb);
-            }
-            __syncthreads();
-            for (int32_t t = threadIdx.x; t < nseg; t += blockDim.x)
-            {
-                const int32_t a = max(cx.beg[t], w0), b = min(cx.beg[t + 1], w0 + wn);
-                if (a >= b) continue;
-                float acc = 0.f;
-                for (int32_t i = a; i < b; ++i) acc += s_contrib[i - w0];
-                s_seg[t] += acc;
-            }
-            __syncthreads();
-        }
-        for (int32_t t = threadIdx.x; t < nseg; t += blockDim.x) seg_partial[cx.k[t]] = s_seg[t];
-    }
-}
-
-// Backward: persistent workgroups of 4 waves; per wave and tile of 32 samples, recompute the forward, back-propagate
-// on the matrix cores, write dL/dfeature per sample (for the LDS scatter), and accumulate the parameter gradient
+// Backward of the FP32 form with silu hidden layers: persistent workgroups of 4 waves; per wave and tile of 32 samples,
+// recompute the forward, back-propagate on the FP32 matrix cores, write dL/dfeature per sample (for the LDS scatter), and accumulate the parameter gradient
 // with products over the tile's samples (staged through LDS as [row][sample]). Each wave writes its own slice of the
 // partials (summed later in a fixed order).
-template <typename P, int H, int ACT>
+template <int H>
 __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const float* __restrict__ params,
-                                                  const void* grid_lowp, const float* grad_proj, float* dfeat,
-                                                  float4* sgc, unsigned int* dmax, float* partials, int32_t P_total)
+                                                  const float* grad_proj, float* dfeat, float4* sgc,
+                                                  unsigned int* dmax, float* partials, int32_t P_total)
 {
+    typedef PrecF32 P;
     constexpr int MT = H / 32, C = 8;
     __shared__ WeightLDS<P, H> w;
     __shared__ ChunkCtx cx;
@@ -840,7 +774,7 @@ __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const floa
         load_chunk_ctx(g, p, q0, q1, base, grad_proj, cx);
         NodeBox nb;
         node_bounds(g, g.seg_node[p.perm[q0]], nb);
-        const void* ngrid = node_grid_ptr(g, grid_lowp, P::kBF16, slot);
+        const void* ngrid = node_grid_ptr(g, nullptr, false, slot);
         __syncthreads();
         const int32_t nsamp = cx.beg[nseg];
         float cmax = 0.f;  // this chunk's
@@ -852,16 +786,12 @@ __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const floa
             // pairs of tiles per wave (fetch_pair)
             auto tile = [&](int32_t i, const float (&x4)[4], float gy) {
                 const bool valid = i < wn;
-                const f32x16 dx = tile_backward_mfma<P, H, ACT>(w, x4, gy, valid, NEAT_ACT_SOFTPLUS, g.beta, sb, acc);
+                const f32x16 dx = tile_backward_mfma<P, H, NEAT_ACT_SILU>(w, x4, gy, valid, NEAT_ACT_SOFTPLUS, g.beta, sb, acc);
                 if (valid)
                 {
-                    // FP32 form: [2][S][4] (channel halves); BF16 form: [S][8] BF16, this lane's 4 channels
-                    if constexpr (P::kBF16)
-                        *reinterpret_cast<uint2*>(reinterpret_cast<unsigned short*>(dfeat) + (base + w0 + i) * 8 +
-                                                  4 * hg) = bf16x4_bits(dx[0], dx[1], dx[2], dx[3]);
-                    else
-                        *reinterpret_cast<float4*>(dfeat + ((int64_t)hg * g.S + base + w0 + i) * 4) =
-                            make_float4(dx[0], dx[1], dx[2], dx[3]);
+                    // [2][S][4]: channel halves
+                    *reinterpret_cast<float4*>(dfeat + ((int64_t)hg * g.S + base + w0 + i) * 4) =
+                        make_float4(dx[0], dx[1], dx[2], dx[3]);
                     cmax = fmaxf(cmax, fmaxf(fmaxf(fabsf(dx[0]), fabsf(dx[1])), fmaxf(fabsf(dx[2]), fabsf(dx[3]))));
                 }
             };
@@ -977,13 +907,12 @@ int node_workgroups()
 int bw1_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::min<int64_t>(z.max1, 2048)); }
 // matrix-core backward: persistent workgroups of 4 waves, one partial slice per wave
 int mfma_bwd_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::min<int64_t>(z.max1, 256)); }
-// split forward: persistent workgroups, one per CU (their LDS)
-int split_fwd_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::min<int64_t>(z.max1, 256)); }
-int mfma_fwd_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::min<int64_t>(z.max1, 1024)); }
+// split and silu forward: persistent workgroups, one per CU (their LDS)
+int fwd_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::min<int64_t>(z.max1, 256)); }
 
 size_t partials_bytes(const ProjSizes& z)
 {
-    size_t slices = std::max<size_t>({(size_t)bw1_workgroups(z), (size_t)mfma_bwd_workgroups(z) * 4,
+    size_t slices = std::max<size_t>({(size_t)bw1_workgroups(z), (size_t)bf16_bwd_slices(mfma_bwd_workgroups(z)),
                                       (size_t)kNodeWGMax * kNodeWaves});
     return (slices * z.P * 4 + 255) / 256 * 256;
 }
@@ -1137,24 +1066,19 @@ int launch_fwd_mfma(hipStream_t s, const Args& a, const Plan& p, float* seg_part
 {
     if constexpr (!P::kBF16)
     {
-        NEAT_REQUIRE(launch_split_fwd(s, H, a.act, split_fwd_workgroups(a.z), a.g, p, a.params, seg_partial,
+        NEAT_REQUIRE(launch_split_fwd(s, H, a.act, fwd_workgroups(a.z), a.g, p, a.params, seg_partial,
                                       sample_out) == 0,
                      "k_split_fwd launch failed");
     }
     else
     {
-        const unsigned grid = (unsigned)mfma_fwd_workgroups(a.z);
         if (a.relu16)
-        {
             NEAT_REQUIRE(launch_mfma_fwd_relu(s, H, a.g, p, a.params, a.grid_bf16, seg_partial, sample_out) == 0,
                          "k_mfma_fwd_relu launch failed");
-            return NEAT_OK;
-        }
-        if (a.act == NEAT_ACT_RELU)
-            k_mfma_fwd<H, NEAT_ACT_RELU><<<grid, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, seg_partial, sample_out);
         else
-            k_mfma_fwd<H, NEAT_ACT_SILU><<<grid, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, seg_partial, sample_out);
-        NEAT_LAUNCHED();
+            NEAT_REQUIRE(launch_bf16_fwd(s, H, fwd_workgroups(a.z), a.g, p, a.params, a.grid_bf16, seg_partial,
+                                         sample_out) == 0,
+                         "k_bf16_fwd launch failed");
     }
     return NEAT_OK;
 }
@@ -1230,12 +1154,12 @@ int launch_bw_valu(hipStream_t s, const Args& a, const Plan& p, const BwdBufs& b
 template <typename P, int H>
 int launch_bw_mfma(hipStream_t s, const Args& a, const Plan& p, const BwdBufs& b, int stage)
 {
-    // BF16 with relu hidden layers runs k_mfma_bwd_relu (node-resident: p.nwg workgroups of kNodeWaves waves)
+    // BF16 with relu hidden layers runs k_mfma_bwd_relu (node-resident: p.nwg workgroups of kNodeWaves waves), with silu
+    // k_bf16_bwd; FP32 with relu k_split_bwd (the masks it folds into its products need relu), with silu k_mfma_bwd
     const bool relu16 = P::kBF16 && a.relu16;
-    // FP32 with relu hidden layers runs k_split_bwd (the masks it folds into its products need relu)
     const bool relu32 = !P::kBF16 && a.act == NEAT_ACT_RELU;
     const int nwg     = mfma_bwd_workgroups(a.z);
-    const int slices  = relu16 ? p.nwg * kNodeWaves : (relu32 ? nwg : nwg * 4);
+    const int slices  = relu16 ? p.nwg * kNodeWaves : (P::kBF16 ? bf16_bwd_slices(nwg) : (relu32 ? nwg : nwg * 4));
     const int Ptot    = a.m.nparams();
     if (stage == 1)
     {
@@ -1250,12 +1174,10 @@ int launch_bw_mfma(hipStream_t s, const Args& a, const Plan& p, const BwdBufs& b
         }
         if constexpr (P::kBF16)
         {
-            if (a.act == NEAT_ACT_RELU)
-                k_mfma_bwd<P, H, NEAT_ACT_RELU><<<nwg, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, b.grad_proj,
-                                                                     b.dfeat, b.sgc, b.dmax, b.partials, Ptot);
-            else
-                k_mfma_bwd<P, H, NEAT_ACT_SILU><<<nwg, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, b.grad_proj,
-                                                                     b.dfeat, b.sgc, b.dmax, b.partials, Ptot);
+            const int rc = launch_bf16_bwd(s, H, nwg, a.g, p, a.params, a.grid_bf16, b.grad_proj, b.dfeat, b.sgc, b.dmax,
+                                           b.partials, Ptot);
+            NEAT_REQUIRE(rc == 0, "k_bf16_bwd launch failed");
+            return NEAT_OK;
         }
         else
         {
@@ -1266,8 +1188,7 @@ int launch_bw_mfma(hipStream_t s, const Args& a, const Plan& p, const BwdBufs& b
                 NEAT_REQUIRE(rc == 0, "k_split_bwd launch failed");
                 return NEAT_OK;
             }
-            k_mfma_bwd<P, H, NEAT_ACT_SILU><<<nwg, 256, 0, s>>>(a.g, p, a.params, a.grid_bf16, b.grad_proj, b.dfeat,
-                                                                 b.sgc, b.dmax, b.partials, Ptot);
+            k_mfma_bwd<H><<<nwg, 256, 0, s>>>(a.g, p, a.params, b.grad_proj, b.dfeat, b.sgc, b.dmax, b.partials, Ptot);
         }
         NEAT_LAUNCHED();
         return NEAT_OK;

@@ -690,4 +690,14 @@ int launch_split_bwd(hipStream_t s, int H, int workgroups, const ProjGeom& g, co
                      const float* grad_proj, float* dfeat, float4* sgc, unsigned int* dmax, float* partials,
                      int32_t P_total);
 
+// ---- silu BF16 forward and backward (projector_silu.hip) -----------------------------------------------------------
+int launch_bf16_fwd(hipStream_t s, int H, int workgroups, const ProjGeom& g, const Plan& p, const float* params,
+                    const void* grid_bf16, float* seg_partial, float* sample_out);
+
+// Launches k_bf16_bwd<H> (H = 32 or 64); bf16_bwd_slices(workgroups) parameter-gradient slices.
+int bf16_bwd_slices(int workgroups);
+int launch_bf16_bwd(hipStream_t s, int H, int workgroups, const ProjGeom& g, const Plan& p, const float* params,
+                    const void* grid_bf16, const float* grad_proj, float* dfeat, float4* sgc, unsigned int* dmax,
+                    float* partials, int32_t P_total);
+
 }  // namespace neat

@@ -114,3 +114,28 @@ def test_projector_against_vector_form(rays, H, act):
         out.append([pj.forward(), *pj.backward(gproj)])
     for a, b in zip(*out):
         assert rel(a, b.double()) <= 1e-5  # both within 1e-5 of the oracle's FP32 form; a unit at zero may flip
+
+
+@pytest.mark.parametrize("H", [32, 64])
+@pytest.mark.parametrize("rays", [1, 3, 70, 4001])
+def test_bf16_silu_projector_edges(rays, H):
+    """The BF16 form with silu against the FP32 form: 1e-3 for projections and 1e-2 for gradients, the bars the BF16
+    arithmetic is held to against FP64."""
+    print("case: bf16 silu projector", rays, H, flush=True)
+    cfg = W.C1
+    sc = W.make_scene(cfg, seed=1)
+    ds = pipeline.to_device(sc, cfg)
+    ds.params = torch.from_numpy(W.decoder_params(8, H, 1, 1, 4)).to(DEV)
+    ds.mlp = dict(ds.mlp, hidden=H, act="silu")
+    o, d = W.batch_rays(cfg, rays, seed=rays)
+    to, td = torch.from_numpy(o).to(DEV), torch.from_numpy(d).to(DEV)
+    td[0] = -to[0] / to[0].norm()  # at least one ray through the volume
+    segs = pipeline.sample(ds, to, td, jitter=True, seed=2, emit=False)
+    gproj = torch.randn(rays, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1))
+    out = []
+    for precision in ("bf16", "fp32"):
+        pj = ops.Projector(ds.pos_min, ds.pos_max, ds.prefix, to, td, segs, ds.grid, ds.params, ds.mlp, True, 2,
+                           precision=precision)
+        out.append([pj.forward(), *pj.backward(gproj)])
+    for a, b, bar in zip(*out, (1e-3, 1e-2, 1e-2)):
+        assert rel(a, b.double()) <= bar
