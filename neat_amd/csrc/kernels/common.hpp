@@ -192,5 +192,8 @@ __device__ __forceinline__ float act_d(int a, float x, float beta)
 // ---- exclusive scan of int64 in place: a[0..n) counts -> a[0..n] offsets (a[n] = total) --------------------------------
 size_t scan_workspace_bytes(int64_t n);
 int exclusive_scan_i64(hipStream_t stream, int64_t* a, int64_t n, void* workspace, size_t workspace_bytes);
+// two arrays of the same length (together when the workspace holds scan_workspace_bytes(n) twice, one after the other
+// with less)
+int exclusive_scan2_i64(hipStream_t stream, int64_t* a, int64_t* b, int64_t n, void* workspace, size_t workspace_bytes);
 
 }  // namespace neat

@@ -35,18 +35,10 @@ __global__ void __launch_bounds__(256) k_plan_keys(ProjGeom g, int32_t* keys, in
     vals[k]      = (int32_t)k;
 }
 
-__global__ void __launch_bounds__(256) k_plan_counts(ProjGeom g, const int32_t* perm, int64_t* nm_soff)
+// First position of the sorted keys in [lo, K) with key >= s.
+__device__ __forceinline__ int64_t lower_key(const int32_t* skeys, int64_t lo, int64_t K, int64_t s)
 {
-    int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < g.K) nm_soff[q] = g.seg_count[perm[q]];
-}
-
-__global__ void __launch_bounds__(256) k_plan_slots(ProjGeom g, const int32_t* skeys, Plan p)
-{
-    int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s > g.N) return;
-    // lower bound of s in the sorted keys
-    int64_t lo = 0, hi = g.K;
+    int64_t hi = K;
     while (lo < hi)
     {
         int64_t mid = (lo + hi) >> 1;
@@ -55,18 +47,21 @@ __global__ void __launch_bounds__(256) k_plan_slots(ProjGeom g, const int32_t* s
         else
             hi = mid;
     }
-    p.slot_begin[s] = (int32_t)lo;
+    return lo;
 }
 
-// Forward / backward-pass-1 chunks are cut by the cost samples + kSegCost x segments, in steps of kFwdChunk: a
-// chunk then holds fewer than kFwdChunk / kSegCost + 1 segments and fewer than kFwdChunk samples plus its last
-// segment's.
-__global__ void __launch_bounds__(256) k_plan_chunk_counts(ProjGeom g, Plan p)
+// Each slot's node-major segment range and chunk counts (nm_soff scanned). Forward / backward-pass-1 chunks are cut by
+// the cost samples + kSegCost x segments, in steps of kFwdChunk: a chunk then holds fewer than kFwdChunk / kSegCost + 1
+// segments and fewer than kFwdChunk samples plus its last segment's. Thread 0 also clears the reduction list's count.
+__global__ void __launch_bounds__(256) k_plan_slots(ProjGeom g, const int32_t* skeys, Plan p)
 {
-    int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= g.N) return;
-    const int32_t sb = p.slot_begin[s], se = p.slot_begin[s + 1];
-    int64_t n       = p.nm_soff[se] - p.nm_soff[sb];
+    const int64_t sb = lower_key(skeys, 0, g.K, s), se = lower_key(skeys, sb, g.K, s + 1);
+    p.slot_begin[s] = (int32_t)sb;
+    if (s == g.N - 1) p.slot_begin[g.N] = (int32_t)se;
+    if (s == 0) *p.nredo = 0;
+    const int64_t n = p.nm_soff[se] - p.nm_soff[sb];
     p.chunk_off1[s] = (n + (int64_t)kSegCost * (se - sb) + kFwdChunk - 1) / kFwdChunk;
     p.chunk_off2[s] = (n + p.chunk2 - 1) / p.chunk2;
 }
@@ -102,12 +97,20 @@ __device__ __forceinline__ int32_t lower_cost(const int64_t* nm_soff, int32_t sb
 
 // One thread per chunk. Scatter chunk r of a slot covers the slot's segments whose first sample lies in
 // [r*T, (r+1)*T) (relative to the slot's first sample); forward chunk r those whose cost lies in that range.
-// Threads [0, max1) fill forward chunks, [max1, max1 + max2) scatter chunks.
+// Threads [0, max1) fill forward chunks, [max1, max1 + max2) scatter chunks, [max1 + max2, max1 + max2 + N) list the
+// slots the scatter's reduction visits: those with no scatter chunk or with several.
 __global__ void __launch_bounds__(256) k_plan_chunks(ProjGeom g, Plan p)
 {
     int64_t i       = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool pass1 = i < p.max1;
     if (!pass1) i -= p.max1;
+    if (!pass1 && i >= p.max2)
+    {
+        const int64_t slot = i - p.max2;
+        if (slot < g.N && p.chunk_off2[slot + 1] - p.chunk_off2[slot] != 1)
+            p.redo_slots[atomicAdd(p.nredo, 1)] = (int32_t)slot;
+        return;
+    }
     const int64_t* off = pass1 ? p.chunk_off1 : p.chunk_off2;
     if (i >= (pass1 ? p.max1 : p.max2) || i >= off[g.N]) return;
     // slot owning chunk i: last s with off[s] <= i
@@ -141,11 +144,14 @@ __global__ void __launch_bounds__(256) k_plan_chunks(ProjGeom g, Plan p)
     (pass1 ? p.chunk1_q1 : p.chunk2_q1)[i]     = q1;
 }
 
-// Per-segment records in node-major order (make_record), after the sort.
-__global__ void __launch_bounds__(256) k_plan_records(ProjGeom g, Plan p)
+// Per-segment records in node-major order (make_record), after the sort, with the sample counts (for the scan into
+// nm_soff); and the segments' partial sums cleared: those whose node has no valid slot are in no chunk and stay zero.
+__global__ void __launch_bounds__(256) k_plan_records(ProjGeom g, Plan p, float* seg_partial)
 {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < g.K) make_record(g, p, q);
+    if (q >= g.K) return;
+    p.nm_soff[q]   = make_record(g, p, q);
+    seg_partial[q] = 0.f;
 }
 
 // Node-resident workgroup ranges: workgroup b takes the forward chunks whose first segment starts at a cost
@@ -723,14 +729,6 @@ __global__ void __launch_bounds__(256) k_proj_bw2_reduce(ProjGeom g, Plan p, int
     }
 }
 
-// The slots the reduction visits: those with no scatter chunk or with several.
-__global__ void __launch_bounds__(256) k_plan_redo(ProjGeom g, Plan p)
-{
-    const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= g.N) return;
-    if (p.chunk_off2[slot + 1] - p.chunk_off2[slot] != 1) p.redo_slots[atomicAdd(p.nredo, 1)] = (int32_t)slot;
-}
-
 __global__ void __launch_bounds__(256) k_fill_f32(float* p, int64_t n, float v)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -880,8 +878,8 @@ Layout proj_layout(const ProjSizes& z)
     L.add(4 * z.K);                       // 7 keys (sort in)
     L.add(4 * z.K);                       // 8 keys (sorted)
     L.add(4 * z.K);                       // 9 vals (sort in)
-    L.add(std::max<size_t>(z.sort_temp, scan_workspace_bytes(z.K + 1)));  // 10 sort / scan temp
-    L.add(4 * z.K);                       // 11 seg_partial (forward)
+    L.add(std::max<size_t>(z.sort_temp, 2 * scan_workspace_bytes(std::max(z.K, z.N) + 1)));  // 10 sort / scan temp
+    L.add(4 * z.K);                       // 11 seg_partial (cleared by the plan, written by the forward)
     L.add(4 * (size_t)z.P);               // 12 transposed decoder params
     L.add(4 * (size_t)z.S * z.C);         // 13 dfeat ([S][C]; FP32 matrix-core: [C/4][S][4]; BF16: [S][8] BF16)
     L.add(16 * (size_t)z.S);              // 14 grid coordinates per sample, matrix-core backward (BF16: packed, 8 B)
@@ -1517,32 +1515,16 @@ extern "C"
             size_t tmp = z.sort_temp;
             NEAT_HIP(hipcub::DeviceRadixSort::SortPairs(temp, tmp, keys, skeys, vals, p.perm, (int)z.K, 0, end_bit,
                                                         s));
-            k_plan_records<<<grid_for(z.K, 256), 256, 0, s>>>(a.g, p);
-            NEAT_LAUNCHED();
-            k_plan_counts<<<grid_for(z.K, 256), 256, 0, s>>>(a.g, p.perm, p.nm_soff);
+            k_plan_records<<<grid_for(z.K, 256), 256, 0, s>>>(a.g, p, reinterpret_cast<float*>(region(ws, z, 11)));
             NEAT_LAUNCHED();
         }
         if ((st = exclusive_scan_i64(s, p.nm_soff, z.K, temp, temp_sz))) return st;
-        if (z.K > 0)
-        {
-            k_plan_slots<<<grid_for(z.N + 1, 256), 256, 0, s>>>(a.g, skeys, p);
-            NEAT_LAUNCHED();
-        }
-        else
-        {
-            NEAT_HIP(hipMemsetAsync(p.slot_begin, 0, (size_t)(z.N + 1) * sizeof(int32_t), s));
-        }
-        k_plan_chunk_counts<<<grid_for(z.N, 256), 256, 0, s>>>(a.g, p);
+        k_plan_slots<<<grid_for(z.N, 256), 256, 0, s>>>(a.g, skeys, p);
         NEAT_LAUNCHED();
-        if ((st = exclusive_scan_i64(s, p.chunk_off1, z.N, temp, temp_sz))) return st;
-        if ((st = exclusive_scan_i64(s, p.chunk_off2, z.N, temp, temp_sz))) return st;
-        k_plan_chunks<<<grid_for(z.max1 + z.max2, 256), 256, 0, s>>>(a.g, p);
+        if ((st = exclusive_scan2_i64(s, p.chunk_off1, p.chunk_off2, z.N, temp, temp_sz))) return st;
+        k_plan_chunks<<<grid_for(z.max1 + z.max2 + z.N, 256), 256, 0, s>>>(a.g, p);
         NEAT_LAUNCHED();
         k_plan_wg<<<grid_for(p.nwg + 1, 256), 256, 0, s>>>(a.g, p);
-        NEAT_LAUNCHED();
-        k_fill_f32<<<1, 64, 0, s>>>(reinterpret_cast<float*>(p.nredo), 1, 0.f);  // zero bits
-        NEAT_LAUNCHED();
-        k_plan_redo<<<grid_for(z.N, 256), 256, 0, s>>>(a.g, p);
         NEAT_LAUNCHED();
         return NEAT_OK;
     }
@@ -1560,9 +1542,6 @@ extern "C"
         float* seg_partial = reinterpret_cast<float*>(region(ws, a.z, 11));
         if (a.z.K > 0)
         {
-            // segments whose node has no valid slot are in no chunk: they contribute zero
-            k_fill_f32<<<grid_for(a.z.K, 256), 256, 0, s>>>(seg_partial, a.z.K, 0.f);
-            NEAT_LAUNCHED();
             if ((st = dispatch_fwd(s, a, p, seg_partial))) return st;
         }
         if (x->num_rays > 0)
@@ -1589,8 +1568,6 @@ extern "C"
         hipStream_t s      = as_stream(stream);
         Plan p             = plan_view(ws, a.z);
         float* seg_partial = reinterpret_cast<float*>(region(ws, a.z, 11));
-        k_fill_f32<<<grid_for(a.z.K, 256), 256, 0, s>>>(seg_partial, a.z.K, 0.f);
-        NEAT_LAUNCHED();
         if (a.precision == NEAT_PREC_BF16)
             st = a.m.hidden == 64 ? launch_fwd_mfma<PrecBF16, 64>(s, a, p, seg_partial, values)
                                   : launch_fwd_mfma<PrecBF16, 32>(s, a, p, seg_partial, values);

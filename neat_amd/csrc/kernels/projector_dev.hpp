@@ -409,8 +409,8 @@ struct ChunkCtx
 };
 
 // Record of the segment at node-major position q (k = perm[q]): what ChunkCtx holds, computed with the same
-// operations as sample_geo and proposal_cell so every derived value has the same bits.
-__device__ inline void make_record(const ProjGeom& g, const Plan& p, int64_t q)
+// operations as sample_geo and proposal_cell so every derived value has the same bits. Returns the sample count.
+__device__ inline int32_t make_record(const ProjGeom& g, const Plan& p, int64_t q)
 {
     const int32_t k   = p.perm[q];
     const int32_t ray = g.seg_ray[k];
@@ -439,6 +439,7 @@ __device__ inline void make_record(const ProjGeom& g, const Plan& p, int64_t q)
     p.rec_dt[q] = make_float4(g.rd[3 * (int64_t)ray], g.rd[3 * (int64_t)ray + 1], g.rd[3 * (int64_t)ray + 2], tmax);
     p.rec_i[q]  = make_int4(k, ray, (int32_t)(k - g.ray_seg_offset[ray]), n);
     p.rec_h[q]  = make_uint4((uint32_t)hr, (uint32_t)(hr >> 32), kind, __float_as_uint(step));
+    return n;
 }
 
 __device__ inline void load_chunk_ctx(const ProjGeom& g, const Plan& p, int32_t q0, int32_t q1, int64_t base,

@@ -477,7 +477,7 @@ static int scratch_addr(void** out)
 
 extern "C"
 {
-    size_t neat_raysample_workspace_bytes(int64_t num_rays) { return scan_workspace_bytes(num_rays); }
+    size_t neat_raysample_workspace_bytes(int64_t num_rays) { return 2 * scan_workspace_bytes(num_rays); }
 
     size_t neat_raysample_scratch_bytes(int64_t num_rays, int32_t max_depth)
     {
@@ -510,9 +510,7 @@ extern "C"
                                                          ray_seg_offset, ray_sample_offset, max_per_ray);
             NEAT_LAUNCHED();
         }
-        st = exclusive_scan_i64(s, ray_seg_offset, R, workspace, workspace_bytes);
-        if (st) return st;
-        return exclusive_scan_i64(s, ray_sample_offset, R, workspace, workspace_bytes);
+        return exclusive_scan2_i64(s, ray_seg_offset, ray_sample_offset, R, workspace, workspace_bytes);
     }
 
     int neat_raysample_compact(neat_stream_t stream, const float* pmin, const float* pmax, const uint8_t* flags,
@@ -566,9 +564,7 @@ extern "C"
                                                           max_per_ray);
             NEAT_LAUNCHED();
         }
-        st = exclusive_scan_i64(s, ray_seg_offset, R, workspace, workspace_bytes);
-        if (st) return st;
-        return exclusive_scan_i64(s, ray_sample_offset, R, workspace, workspace_bytes);
+        return exclusive_scan2_i64(s, ray_seg_offset, ray_sample_offset, R, workspace, workspace_bytes);
     }
 
     int neat_raysample_count_noalloc(neat_stream_t stream, const float* pmin, const float* pmax,
