@@ -137,6 +137,9 @@ __device__ __forceinline__ void traverse(const TreeArgs& T, const float o[3], co
     }
 }
 
+// LDS writes of the wave's lanes before this are seen by its reads after
+__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
+
 __device__ __forceinline__ void load_ray(const float* ro, const float* rd, int64_t r, float o[3], float d[3])
 {
 #pragma unroll
@@ -253,8 +256,8 @@ __global__ void __launch_bounds__(128) k_ray_segments(TreeArgs T, const float* r
     }
 }
 
-// Single-walk sampler: segment i of ray r goes to column entry i * R + r of a scratch of `cap` entries per ray
-// (four columns: node, count, tmin, tmax), with the ray's segment and sample counts; once the offsets are known,
+// Single-walk sampler: segment i of ray r goes to entry i * R + r of a scratch of `cap` entries per ray (four arrays:
+// node, count, tmin, tmax; neighbouring rays are neighbouring lanes) or, when a wave walks a ray, to r * cap + i, with the ray's segment and sample counts; once the offsets are known,
 // k_ray_rewalk walks the rays with more than `cap` segments again straight into the canonical list and k_ray_compact
 // copies the scratch of the others.
 struct RayScratch
@@ -264,6 +267,7 @@ struct RayScratch
     float* tmin;
     float* tmax;
     int64_t cap;
+    int64_t ray_stride, seg_stride;
 };
 
 __global__ void __launch_bounds__(128) k_ray_walk(TreeArgs T, const float* ro, const float* rd, int64_t R,
@@ -275,10 +279,164 @@ __global__ void __launch_bounds__(128) k_ray_walk(TreeArgs T, const float* ro, c
     float o[3], d[3];
     load_ray(ro, rd, r, o, d);
     int64_t nk, ns;
-    walk_sorted(T, o, d, max_spn, sc.node, sc.count, sc.tmin, sc.tmax, r, R, sc.cap, nk, ns);
+    walk_sorted(T, o, d, max_spn, sc.node, sc.count, sc.tmin, sc.tmax, r * sc.ray_stride, sc.seg_stride, sc.cap, nk,
+                ns);
     nseg[r]  = nk;
     nsamp[r] = ns;
     if (max_per_ray) atomicMax(max_per_ray, (int32_t)ns);
+}
+
+// One wave per ray, for batches too small to fill the chip with one thread per ray: the octree level by level, the lanes
+// testing the children of the level's hit nodes that have active descendants. A child is tested exactly when the
+// stackless walk would visit it (its parent is hit and has an active descendant), with the same box (halved from the
+// parent's) and the same slab test, so the segments are the same; they are put in canonical order by ranking each
+// against the others. A ray with more than kCoopSegs segments, or more than kCoopNodes nodes to expand on one level
+// (rays along faces touch both sides of them), is walked by one lane instead.
+//
+// The walk is a chain of dependent steps, about 300 per ray in a depth-5 tree, whose latency a small batch does not
+// hide; here it is one round per 64 children. A thread per ray costs less work in all, hence the limit in coop_rays
+// (both measured there).
+constexpr int kCoopWaves = 4;
+constexpr int kCoopNodes = 128;
+constexpr int kCoopSegs  = 128;
+
+struct CoopList
+{
+    int32_t node[kCoopNodes];
+    float mn[3][kCoopNodes], mx[3][kCoopNodes];
+};
+
+__global__ void __launch_bounds__(64 * kCoopWaves) k_ray_coop(TreeArgs T, const float* ro, const float* rd, int64_t R,
+                                                              int32_t max_spn, RayScratch sc, int64_t* nseg,
+                                                              int64_t* nsamp, int32_t* max_per_ray)
+{
+    __shared__ CoopList s_list[kCoopWaves][2];
+    __shared__ int32_t s_node[kCoopWaves][kCoopSegs], s_cnt[kCoopWaves][kCoopSegs];
+    __shared__ float s_tmin[kCoopWaves][kCoopSegs], s_tmax[kCoopWaves][kCoopSegs];
+    const int l = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t r = (int64_t)blockIdx.x * kCoopWaves + wave;
+    if (r >= R) return;  // the whole wave; nothing below synchronises across waves
+    float o[3], d[3];
+    load_ray(ro, rd, r, o, d);
+    const uint64_t below = l == 0 ? 0 : (~(uint64_t)0 >> (64 - l));
+    int32_t k = 0, ns = 0, m = 0, cur = 0;  // segments, samples (this lane's), nodes to expand, the list that holds them
+    bool over = false;
+    // a hit node: its segment if it is active, its place on the next level's list if it is to be expanded
+    auto visit = [&](bool hit, int32_t n, uint32_t f, const float mn[3], const float mx[3], const Hit& h, int32_t& next) {
+        const bool seg   = hit && (f & 1) && !((double)(h.tmax - h.tmin) < 1e-5);
+        const uint64_t a = __ballot(seg);
+        if (seg)
+        {
+            const int32_t at = k + __popcll(a & below);
+            if (at < kCoopSegs)
+            {
+                const int32_t c  = segment_count(mn, mx, h.tmin, h.tmax, max_spn);
+                s_node[wave][at] = n;
+                s_tmin[wave][at] = h.tmin;
+                s_tmax[wave][at] = h.tmax;
+                s_cnt[wave][at]  = c;
+                ns += c;
+            }
+        }
+        k += __popcll(a);
+        const bool desc  = hit && (f & 2) && n < T.first_leaf;  // never leave the node table
+        const uint64_t e = __ballot(desc);
+        if (desc)
+        {
+            const int32_t at = next + __popcll(e & below);
+            if (at < kCoopNodes)
+            {
+                CoopList& L = s_list[wave][cur ^ 1];
+                L.node[at]  = n;
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                {
+                    L.mn[q][at] = mn[q];
+                    L.mx[q][at] = mx[q];
+                }
+            }
+        }
+        next += __popcll(e);
+    };
+    {
+        const float mn[3] = {T.pmin[0], T.pmin[1], T.pmin[2]}, mx[3] = {T.pmax[0], T.pmax[1], T.pmax[2]};
+        const uint32_t f = T.flags[0];
+        Hit h{false, 0.f, 0.f};
+        if (f && l == 0) h = slab_test(mn, mx, o, d);
+        visit(h.hit, 0, f, mn, mx, h, m);
+    }
+    while (m > 0 && !over)
+    {
+        cur ^= 1;
+        wave_fence();
+        const CoopList& L = s_list[wave][cur];
+        int32_t next      = 0;
+        for (int32_t b = 0; b < 8 * m; b += 64)
+        {
+            const int32_t i = b + l, pi = min(i >> 3, m - 1), c = i & 7;
+            const int32_t n = 8 * L.node[pi] + 1 + c;
+            const uint32_t f = i < 8 * m ? T.flags[n] : 0u;
+            float mn[3], mx[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+            {
+                const float a = L.mn[q][pi], e = L.mx[q][pi], ce = (a + e) * 0.5f;
+                mn[q] = ((c >> q) & 1) ? ce : a;
+                mx[q] = ((c >> q) & 1) ? e : ce;
+            }
+            Hit h{false, 0.f, 0.f};
+            if (f) h = slab_test(mn, mx, o, d);
+            visit(h.hit, n, f, mn, mx, h, next);
+        }
+        m    = next;
+        over = m > kCoopNodes || k > kCoopSegs;
+    }
+    over = over || k > kCoopSegs;
+    if (over)
+    {
+        if (l == 0)
+        {
+            int64_t nk, nn;
+            walk_sorted(T, o, d, max_spn, sc.node, sc.count, sc.tmin, sc.tmax, r * sc.ray_stride, sc.seg_stride, sc.cap,
+                        nk, nn);
+            nseg[r]  = nk;
+            nsamp[r] = nn;
+            if (max_per_ray) atomicMax(max_per_ray, (int32_t)nn);
+        }
+        return;
+    }
+    wave_fence();
+    for (int32_t b = 0; b < k; b += 64)
+    {
+        const int32_t i = b + l;
+        if (i < k)
+        {
+            const float t   = s_tmin[wave][i];
+            const int32_t n = s_node[wave][i];
+            int32_t rank    = 0;
+            for (int32_t j = 0; j < k; ++j) rank += seg_less(s_tmin[wave][j], s_node[wave][j], t, n) ? 1 : 0;
+            if (rank < sc.cap)
+            {
+                const int64_t e = r * sc.ray_stride + rank * sc.seg_stride;
+                sc.node[e]      = n;
+                sc.count[e]     = s_cnt[wave][i];
+                sc.tmin[e]      = t;
+                sc.tmax[e]      = s_tmax[wave][i];
+            }
+        }
+    }
+    int64_t total = ns;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) total += __shfl_xor(total, off);
+    if (l == 0)
+    {
+        nseg[r]  = k;
+        nsamp[r] = total;
+        // one atomic per ray on one address would take longer than the walk: rays below the maximum so far skip it
+        if (max_per_ray &&
+            (int32_t)total > __hip_atomic_load(max_per_ray, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax(max_per_ray, (int32_t)total);
+    }
 }
 
 // Rays with more segments than the scratch holds (cap): walked again, straight into the canonical list.
@@ -345,7 +503,7 @@ __global__ void __launch_bounds__(64 * kCompactWaves) k_ray_compact(int64_t R, R
             }
             else
             {
-                const int64_t e = (q - oj) * R + r;
+                const int64_t e = (q - oj) * sc.seg_stride + r * sc.ray_stride;
                 cnt             = sc.count[e];
                 seg_node[q]     = sc.node[e];
                 seg_count[q]    = cnt;
@@ -432,10 +590,26 @@ static int64_t scratch_cap(int32_t max_depth)
     return std::min<int64_t>(c, 128);
 }
 
+// Rays up to which a wave walks a ray (k_ray_coop): a deeper tree makes the chain of one thread's steps longer and gives a
+// wave more to do at a time. Whole sampler in us, wave / thread per ray, for rays drawn over all views and for the
+// consecutive rays of one view (whose threads stay together): uniform depth 2, 64 leaves: 86 / 103 and 83 / 94 at 2,048
+// rays, 95 / 104 and 98 / 87 at 4,099, 126 / 110 and 126 / 106 at 16,384; depth 5, 4096 leaves: 98 / 446 and 112 / 251 at
+// 4,099, 188 / 477 and 165 / 176 at 32,768, 214 / 467 and 160 / 161 at 65,536, 338 / 488 and 260 / 282 at 131,072,
+// 568 / 612 and 532 / 352 at 262,144. The limits are where neither kind loses; between the two trees, a factor of about 3
+// a level.
+static int64_t coop_rays(int32_t max_depth)
+{
+    static constexpr int64_t kRays[] = {2048, 2048, 2048, 6144, 20480, 65536};
+    return kRays[std::min(max_depth, 5)];
+}
+
 static RayScratch scratch_view(void* p, int64_t R, int32_t max_depth)
 {
     RayScratch sc;
     sc.cap        = scratch_cap(max_depth);
+    const bool co = R <= coop_rays(max_depth);
+    sc.ray_stride = co ? sc.cap : 1;
+    sc.seg_stride = co ? 1 : R;
     const size_t n = (size_t)(sc.cap * R);
     char* b       = static_cast<char*>(p);
     sc.node       = reinterpret_cast<int32_t*>(b);
@@ -506,8 +680,13 @@ extern "C"
         if (R > 0)
         {
             TreeArgs T{pmin, pmax, flags, first_leaf(num_nodes)};
-            k_ray_walk<<<grid_for(R, 128), 128, 0, s>>>(T, ro, rd, R, max_spn, scratch_view(scratch, R, max_depth),
-                                                         ray_seg_offset, ray_sample_offset, max_per_ray);
+            const RayScratch sc = scratch_view(scratch, R, max_depth);
+            if (R <= coop_rays(max_depth))
+                k_ray_coop<<<grid_for(R, kCoopWaves), 64 * kCoopWaves, 0, s>>>(T, ro, rd, R, max_spn, sc, ray_seg_offset,
+                                                                               ray_sample_offset, max_per_ray);
+            else
+                k_ray_walk<<<grid_for(R, 128), 128, 0, s>>>(T, ro, rd, R, max_spn, sc, ray_seg_offset,
+                                                             ray_sample_offset, max_per_ray);
             NEAT_LAUNCHED();
         }
         return exclusive_scan2_i64(s, ray_seg_offset, ray_sample_offset, R, workspace, workspace_bytes);
