@@ -135,6 +135,12 @@ int neat_raysample_compact(neat_stream_t stream, const float* node_pos_min, cons
                            size_t scratch_bytes, int64_t num_segments, int32_t* seg_node, int32_t* seg_ray,
                            int32_t* seg_count, float* seg_tmin, float* seg_tmax, int64_t* seg_sample_offset);
 
+/* No counterpart in the reference: the totals that size pass 2, (segments, samples, largest per-ray sample count), in one
+ * trip. `totals` is int64 [3] in pinned host memory; the call returns when they are there, i.e. it waits for the
+ * stream (so it cannot run under graph capture). max_samples_per_ray may be NULL (its entry is then 0). */
+int neat_raysample_totals(neat_stream_t stream, const int64_t* ray_seg_offset, const int64_t* ray_sample_offset,
+                          const int32_t* max_samples_per_ray, int64_t num_rays, int64_t* totals);
+
 /* Pass 3: SampleList columns (HelperStructs.h:168-189) for every sample: t, weight (midpoint cell width),
  * global coordinate o + d*t [S,3] (may be NULL), ray index, index within the ray, node id. jitter != 0 draws the
  * in-cell position from the counter hash of (seed, ray, segment rank, j); jitter == 0 uses the cell midpoint. */

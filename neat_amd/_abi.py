@@ -40,6 +40,7 @@ SIGNATURES = {
                                            _SZ]),
     "neat_raysample_compact": (ctypes.c_int, [_P, _P, _P, _P, _I32, _I32, _P, _P, _I64, _I32, _P, _P, _P, _SZ, _I64,
                                               _P, _P, _P, _P, _P, _P]),
+    "neat_raysample_totals": (ctypes.c_int, [_P, _P, _P, _P, _I64, _P]),
     "neat_raysample_emit": (ctypes.c_int, [_P, _P, _P, _I64, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _I64, _I32, _U64,
                                            _P, _P, _P, _P, _P, _P]),
     "neat_local_samples": (ctypes.c_int, [_P, _P, _P, _I64, _P, _P, _I32, _P]),
@@ -169,8 +170,11 @@ def ptr(t):
 
 
 def stream_ptr(stream=None):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    """hipStream_t of a torch stream, or of the current device's current stream (whose handle is asked for directly: a
+    torch.cuda.Stream object for it costs about 4 us, and an entry point takes one per call)."""
+    if stream is None:
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    return ctypes.c_void_p(stream.cuda_stream)
 
 
 def call(name, *args):

@@ -150,6 +150,16 @@ __device__ __forceinline__ void load_ray(const float* ro, const float* rd, int64
     }
 }
 
+// Written straight to pinned host memory: one launch and one wait in place of two gathers, a launch-sized copy and its
+// wait (about 20 us a sampler call on the host's side).
+__global__ void k_ray_totals(const int64_t* seg_off, const int64_t* samp_off, const int32_t* max_per_ray, int64_t R,
+                             int64_t* totals)
+{
+    totals[0] = seg_off[R];
+    totals[1] = samp_off[R];
+    totals[2] = max_per_ray ? *max_per_ray : 0;
+}
+
 __global__ void k_zero_i32(int32_t* p)
 {
     if (p) *p = 0;
@@ -783,6 +793,23 @@ extern "C"
             T, ro, rd, R, max_spn, ray_seg_offset, ray_sample_offset, seg_node, seg_ray, seg_count, seg_tmin, seg_tmax,
             seg_sample_offset);
         NEAT_LAUNCHED();
+        return NEAT_OK;
+    }
+
+    int neat_raysample_totals(neat_stream_t stream, const int64_t* ray_seg_offset, const int64_t* ray_sample_offset,
+                              const int32_t* max_per_ray, int64_t R, int64_t* totals)
+    {
+        NEAT_REQUIRE(R >= 0 && ray_seg_offset && ray_sample_offset && totals, "neat_raysample_totals: bad arguments");
+        hipPointerAttribute_t at;
+        if (hipPointerGetAttributes(&at, totals) != hipSuccess || at.type != hipMemoryTypeHost)
+        {
+            (void)hipGetLastError();
+            return fail(NEAT_E_ARG, "neat_raysample_totals: totals must be pinned host memory");
+        }
+        hipStream_t s = as_stream(stream);
+        k_ray_totals<<<1, 1, 0, s>>>(ray_seg_offset, ray_sample_offset, max_per_ray, R, totals);
+        NEAT_LAUNCHED();
+        NEAT_HIP(hipStreamSynchronize(s));
         return NEAT_OK;
     }
 

@@ -70,3 +70,20 @@ def test_offsets_over_scan_forms(n):
     assert torch.equal(r["ray_seg_offset"][1:], nseg.cumsum(0)) and int(r["ray_seg_offset"][0]) == 0
     assert torch.equal(r["ray_sample_offset"][1:], nsmp.cumsum(0)) and int(r["ray_sample_offset"][0]) == 0
     assert r["max_samples_per_ray"] == int(nsmp.max())
+
+
+def test_totals_need_pinned_memory():
+    from neat_amd import _abi
+    print("case: sampler totals", flush=True)
+    off = torch.tensor([0, 3, 7], dtype=torch.int64, device=DEV)
+    mx = torch.tensor([4], dtype=torch.int32, device=DEV)
+    out = torch.empty(3, dtype=torch.int64, pin_memory=True)
+    _abi.call("neat_raysample_totals", _abi.stream_ptr(), _abi.ptr(off), _abi.ptr(off), _abi.ptr(mx), 2, _abi.ptr(out))
+    assert out.tolist() == [7, 7, 4]
+    for bad in (torch.empty(3, dtype=torch.int64), torch.empty(3, dtype=torch.int64, device=DEV)):
+        with pytest.raises(_abi.NeatError):
+            _abi.call("neat_raysample_totals", _abi.stream_ptr(), _abi.ptr(off), _abi.ptr(off), _abi.ptr(mx), 2,
+                      _abi.ptr(bad))
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert _abi.stream_ptr().value == side.cuda_stream
