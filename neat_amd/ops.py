@@ -64,7 +64,7 @@ def raysample(pos_min, pos_max, flags, max_depth, origin, direction, max_spn, ji
     tot = torch.empty(3, dtype=_I64, pin_memory=True)
     call("neat_raysample_totals", s, ptr(seg_off), ptr(samp_off), ptr(maxr), R, ptr(tot))  # waits for the stream
     K, S, maxs = tot.tolist()
-    r = dict(ray_seg_offset=seg_off, ray_sample_offset=samp_off, max_samples_per_ray=maxs, num_samples=S,
+    r = dict(ray_seg_offset=seg_off, ray_sample_offset=samp_off, max_samples_per_ray=maxs,
              seg_node=torch.empty(K, dtype=_I32, device=dev), seg_ray=torch.empty(K, dtype=_I32, device=dev),
              seg_count=torch.empty(K, dtype=_I32, device=dev), seg_tmin=torch.empty(K, dtype=_F32, device=dev),
              seg_tmax=torch.empty(K, dtype=_F32, device=dev), seg_sample_offset=torch.empty(K, dtype=_I64, device=dev))
