@@ -56,8 +56,11 @@ __device__ __forceinline__ int64_t lower_key(const int32_t* skeys, int64_t lo, i
 __global__ void __launch_bounds__(256) k_plan_slots(ProjGeom g, const int32_t* skeys, Plan p)
 {
     const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    // slot s + 1's first segment is the next lane's search; the wave's last lane searches for it itself
+    const int64_t sb = lower_key(skeys, 0, g.K, s);
+    int64_t se       = __shfl_down(sb, 1);
     if (s >= g.N) return;
-    const int64_t sb = lower_key(skeys, 0, g.K, s), se = lower_key(skeys, sb, g.K, s + 1);
+    if ((threadIdx.x & 63) == 63) se = lower_key(skeys, sb, g.K, s + 1);
     p.slot_begin[s] = (int32_t)sb;
     if (s == g.N - 1) p.slot_begin[g.N] = (int32_t)se;
     if (s == 0) *p.nredo = 0;
@@ -380,6 +383,19 @@ __device__ __forceinline__ double fixed_scale(unsigned int maxbits)
     return ldexp(1.0, 45 - e);
 }
 
+// v * scale rounded to the nearest integer (ties to even) for |v * scale| < 2^51: added to 1.5 * 2^52 in one fused
+// multiply-add the integer is the difference of the bit patterns. The general double-to-int64 conversion takes about
+// three times the instructions, and these conversions were most of the scatter's vector work.
+__device__ __forceinline__ unsigned long long to_fixed(float v, double scale)
+{
+    constexpr double kMagic = 6755399441055744.0;
+    const double d = fma((double)v, scale, kMagic);
+    return (unsigned long long)(__double_as_longlong(d) - __double_as_longlong(kMagic));
+}
+
+// The C = 8 form on kept coordinates is bound by vector work and the 64-bit LDS atomics, whose instructions run with
+// about a quarter of the lanes (those that leave a cell at that sample). 53.3 M samples, 4096 grids of 17^3 x 8:
+// 2.18 ms with the general conversion throughout, 1.80 with to_fixed; 4099 rays of the small step: 23 us against 19.
 template <int C>
 __global__ void __launch_bounds__(kScatterThreads) k_proj_bw2(ProjGeom g, Plan p, const float* dfeat,
                                                               const float4* sgc, const unsigned int* dmax,
@@ -430,8 +446,8 @@ __global__ void __launch_bounds__(kScatterThreads) k_proj_bw2(ProjGeom g, Plan p
         const int64_t e2 = min(ns, s2 + L2);
         const double scale = fixed_scale(*dmax);
         const float4* dh   = reinterpret_cast<const float4*>(dfeat) + (int64_t)blockIdx.y * g.S + base;
-        if (s2 < e2)
-        {
+        auto walk = [&](auto fast) {
+            if (s2 >= e2) return;
             int cell = -1;  // (x0 + 1) + (G + 2) ((y0 + 1) + (G + 2) (z0 + 1)) of the current cell (x0 in [-1, G])
             int cx0 = 0, cx1 = 0, cy0 = 0, cy1 = 0, cz0 = 0, cz1 = 0;
             float acc[8][4];
@@ -446,7 +462,10 @@ __global__ void __launch_bounds__(kScatterThreads) k_proj_bw2(ProjGeom g, Plan p
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
                     {
-                        atomicAdd(sq + q * nv + v, (unsigned long long)__double2ll_rn((double)acc[k][q] * scale));
+                        atomicAdd(sq + q * nv + v,
+                                  decltype(fast)::value
+                                      ? to_fixed(acc[k][q], scale)
+                                      : (unsigned long long)__double2ll_rn((double)acc[k][q] * scale));
                         acc[k][q] = 0.f;
                     }
                 }
@@ -505,7 +524,13 @@ __global__ void __launch_bounds__(kScatterThreads) k_proj_bw2(ProjGeom g, Plan p
                 s0 = s1;
             }
             if (cell >= 0) flush();
-        }
+        };
+        // a run of at most 64 samples stays within to_fixed's range: chunks of more than 64 samples per lane (a
+        // segment longer than a chunk) and non-finite gradients take the general conversion
+        if (L2 <= 64 && isfinite(__uint_as_float(*dmax)))
+            walk(std::true_type{});
+        else
+            walk(std::false_type{});
         const int ch0 = 4 * (int)blockIdx.y;
         __syncthreads();
         const bool split = p.chunk_off2[slot + 1] - p.chunk_off2[slot] > 1;
