@@ -113,19 +113,20 @@ constexpr int kEdgeList = 64 * 8;  // gradient entries a wave gathers per side: 
 constexpr int64_t kEdgeDirectBlocks = 4096;  // grid-stride blocks of the fused edge loss (partials per call)
 
 // block total of one double per thread, valid in thread 0, in a fixed order: a butterfly within each wave, then the
-// waves' sums in wave order (blockDim.x = kRedThreads)
+// waves' sums in wave order (blockDim.x = kThreads)
+template <int kThreads = kRedThreads>
 __device__ __forceinline__ double block_total(double v)
 {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    __shared__ double s[kRedThreads / 64];
+    __shared__ double s[kThreads / 64];
     if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
     __syncthreads();
     double t = 0.0;
     if (threadIdx.x == 0)
     {
 #pragma unroll
-        for (int w = 0; w < kRedThreads / 64; ++w) t += s[w];
+        for (int w = 0; w < kThreads / 64; ++w) t += s[w];
     }
     return t;
 }
@@ -136,27 +137,29 @@ __device__ __forceinline__ void block_sum_to(double v, double* out)
     if (threadIdx.x == 0) out[blockIdx.x] = t;
 }
 
-// this thread's share of partials[0, n) (strided by the block), four independent accumulators so the loads overlap
+// The final sums are one block's, bound by the latency of its loads: 1024 threads with 8 loads each in flight take
+// 82,000 partials in 17 us (256 threads with 4: 40).
+constexpr int kSumThreads = 1024;
+
+// this thread's share of partials[0, n) (strided by the block), eight independent accumulators so the loads overlap
 __device__ __forceinline__ double thread_share(const double* partials, int64_t n)
 {
     const int64_t step = blockDim.x;
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+    double a[8] = {};
     int64_t i = threadIdx.x;
-    for (; i + 3 * step < n; i += 4 * step)
+    for (; i + 7 * step < n; i += 8 * step)
     {
-        a0 += partials[i];
-        a1 += partials[i + step];
-        a2 += partials[i + 2 * step];
-        a3 += partials[i + 3 * step];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) a[k] += partials[i + k * step];
     }
-    for (; i < n; i += step) a0 += partials[i];
-    return (a0 + a1) + (a2 + a3);
+    for (; i < n; i += step) a[0] += partials[i];
+    return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
 }
 
-__global__ void __launch_bounds__(kRedThreads) k_sum_partials(const double* partials, int64_t n, double scale,
+__global__ void __launch_bounds__(kSumThreads) k_sum_partials(const double* partials, int64_t n, double scale,
                                                               double* out)
 {
-    const double t = block_total(thread_share(partials, n));
+    const double t = block_total<kSumThreads>(thread_share(partials, n));
     if (threadIdx.x == 0) *out = t * scale;
 }
 
@@ -194,7 +197,8 @@ __global__ void __launch_bounds__(256) k_edge_bwd(const float* f, int64_t P, int
 __device__ __forceinline__ float sgn(float d) { return d > 0.f ? 1.f : (d < 0.f ? -1.f : 0.f); }
 
 // The edge loss straight from the candidate list, without materialising the neighbour rows, their local coordinates
-// or features: lane (candidate, channel quad), so the lanes of a pair read (and, for the gradient, add to) each
+// or features: lane (candidate, kQ channel quads; two where the quads pair up, which halves the work on positions and
+// weights), so the lanes of a pair read (and, for the gradient, add to) each
 // corner's contiguous channel run of a channels-last grid together (16-byte loads when kVec4). Per pair k (row[c],
 // the canonical pair index) the lane samples its channels of both nodes' grids at the shared face point exactly as
 // the grid sample does (same local coordinates, same trilinear weights and corner order), so the features, the
@@ -202,7 +206,7 @@ __device__ __forceinline__ float sgn(float d) { return d > 0.f ? 1.f : (d < 0.f 
 // corners whose weight is exactly zero add nothing and are skipped (face points sit on grid vertices of same-size
 // neighbours). The loss runs per channel as |d| r_k in FP64 (the 1/C of the channel mean cancels against the
 // reference's factor C), per-block partials over a fixed grid-stride assignment, so it is deterministic.
-template <typename I, bool kVec4, bool kLoss, bool kGrad>
+template <typename I, bool kVec4, int kQ, bool kLoss, bool kGrad>
 __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const float* pmin, const float* pmax,
                                                              const int64_t* active_ids, const int64_t* node_slot,
                                                              int64_t num_candidates, int32_t G, const int32_t* other,
@@ -210,7 +214,8 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
                                                              const float* grad_loss, float* grad_grid,
                                                              double* partials)
 {
-    const I quads = (I)((g.C + 3) / 4);
+    constexpr int kCh = 4 * kQ;  // channels of a lane
+    const I quads = (I)((g.C + kCh - 1) / kCh);
     const I total = (I)num_candidates * quads;
     const int64_t P = row[num_candidates];
     float gscale    = 0.f;
@@ -218,11 +223,11 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
         if (P > 0) gscale = (float)((double)*grad_loss * weight / (double)P);
     double acc = 0.0;
     // one lane's pair: its channels' loss terms into acc and their gradients into gv; false when the lane has no pair
-    auto eval = [&](I i, int64_t& sa, int64_t& so, TriLocal& ta, TriLocal& to, float (&gv)[4], int32_t& ch0) -> bool {
+    auto eval = [&](I i, int64_t& sa, int64_t& so, TriLocal& ta, TriLocal& to, float (&gv)[kCh], int32_t& ch0) -> bool {
         const I c       = i / quads;
         const int32_t o = other[c];
         if (o < 0) return false;
-        ch0                = 4 * (int32_t)(i - c * quads);
+        ch0                = kCh * (int32_t)(i - c * quads);
         const Candidate cd = split_candidate<I>(c, G);
         const int32_t node = (int32_t)active_ids[cd.aidx];
         sa = node_slot[node];
@@ -243,31 +248,36 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
         to = trilinear_local(g, uo[0], uo[1], uo[2]);
         const float* ga   = g.grid + sa * g.s0;
         const float* go   = g.grid + so * g.s0;
-        float fa[4] = {0.f, 0.f, 0.f, 0.f}, fo[4] = {0.f, 0.f, 0.f, 0.f};
+        float fa[kCh] = {}, fo[kCh] = {};
         if constexpr (kVec4)
         {
+            // a corner's quads are consecutive 16-byte pieces: their loads hit the lines the first brought in
 #pragma unroll
             for (int k = 0; k < 8; ++k)
-            {
-                const float4 va = *reinterpret_cast<const float4*>(ga + ta.off[k] + ch0);
-                fa[0] += va.x * ta.w[k];
-                fa[1] += va.y * ta.w[k];
-                fa[2] += va.z * ta.w[k];
-                fa[3] += va.w * ta.w[k];
-            }
+#pragma unroll
+                for (int q = 0; q < kQ; ++q)
+                {
+                    const float4 va = *reinterpret_cast<const float4*>(ga + ta.off[k] + ch0 + 4 * q);
+                    fa[4 * q + 0] += va.x * ta.w[k];
+                    fa[4 * q + 1] += va.y * ta.w[k];
+                    fa[4 * q + 2] += va.z * ta.w[k];
+                    fa[4 * q + 3] += va.w * ta.w[k];
+                }
 #pragma unroll
             for (int k = 0; k < 8; ++k)
-            {
-                const float4 vo = *reinterpret_cast<const float4*>(go + to.off[k] + ch0);
-                fo[0] += vo.x * to.w[k];
-                fo[1] += vo.y * to.w[k];
-                fo[2] += vo.z * to.w[k];
-                fo[3] += vo.w * to.w[k];
-            }
+#pragma unroll
+                for (int q = 0; q < kQ; ++q)
+                {
+                    const float4 vo = *reinterpret_cast<const float4*>(go + to.off[k] + ch0 + 4 * q);
+                    fo[4 * q + 0] += vo.x * to.w[k];
+                    fo[4 * q + 1] += vo.y * to.w[k];
+                    fo[4 * q + 2] += vo.z * to.w[k];
+                    fo[4 * q + 3] += vo.w * to.w[k];
+                }
         }
         else
         {
-            for (int j = 0; j < 4 && ch0 + j < g.C; ++j)
+            for (int j = 0; j < kCh && ch0 + j < g.C; ++j)
             {
                 const int32_t co = (ch0 + j) * (int32_t)g.s1;
 #pragma unroll
@@ -277,9 +287,9 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
             }
         }
         const float r = pair_factor(seed, row[c]);
-        const int nch = min(4, g.C - ch0);
+        const int nch = kVec4 ? kCh : min(kCh, g.C - ch0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < kCh; ++j)
         {
             const float d = fa[j] - fo[j];
             if (j < nch)
@@ -293,16 +303,18 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
     const I stride = (I)gridDim.x * (I)blockDim.x;
     if constexpr (kGrad && kVec4)
     {
-        // The gradient's atomics, coalesced: the lanes of a wave append what they add (gradient quad, corner address,
-        // weight; corners of weight zero and quads of zero gradient add nothing) to a list in LDS, and the wave then
-        // takes 16 entries at a time, four lanes to the four consecutive channels of one. Issued from the pairs'
-        // lanes directly, each of an instruction's 64 adds is a request of its own.
+        // The gradient's atomics, coalesced: the lanes of a wave append what they add (gradient quads, corner offset,
+        // weight; corners of weight zero and lanes of zero gradient add nothing) to a list in LDS, and the wave then
+        // takes 64 / kCh entries at a time, kCh lanes to the consecutive channels of one. Issued from the pairs'
+        // lanes directly, each of an instruction's 64 adds is a request of its own. Places in the list come from
+        // ballots: an LDS counter is a round trip per corner, and the offsets it needs alive took 220 registers
+        // (two waves per SIMD) where these take 126.
         // Measured on 4096 random grids of 17^3 x 8 (7.1 M candidates): 2.97 ms with the pairs' lanes adding
-        // directly, 1.04 ms like this (0.61 ms without any add).
-        __shared__ float4 s_gv[kRedThreads];
-        __shared__ int64_t s_off[kRedThreads / 64][kEdgeList];
+        // directly, 1.04 ms with one quad per lane and an LDS counter, 0.86 ms like this.
+        __shared__ float4 s_gv[kRedThreads * kQ];
+        __shared__ int32_t s_off[kRedThreads / 64][kEdgeList];  // within the slot
+        __shared__ int64_t s_base[kRedThreads];
         __shared__ float2 s_w[kRedThreads / 64][kEdgeList];  // weight (signed), lane
-        __shared__ int32_t s_n[kRedThreads / 64];
         const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
         // uniform trip count over the wave: every lane takes part in every list
         for (I i0 = (I)blockIdx.x * (I)blockDim.x + (I)(threadIdx.x & ~63u); i0 < total; i0 += stride)
@@ -310,35 +322,42 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
             const I i = i0 + (I)l;
             int64_t sa = 0, so = 0;
             TriLocal ta, to;
-            float gv[4] = {0.f, 0.f, 0.f, 0.f};
+            float gv[kCh] = {};
             int32_t ch0 = 0;
-            const bool has = i < total && eval(i, sa, so, ta, to, gv, ch0) &&
-                             (gv[0] != 0.f || gv[1] != 0.f || gv[2] != 0.f || gv[3] != 0.f);
-            s_gv[threadIdx.x] = make_float4(gv[0], gv[1], gv[2], gv[3]);
+            bool has = i < total && eval(i, sa, so, ta, to, gv, ch0);
+            bool any = false;
+#pragma unroll
+            for (int q = 0; q < kQ; ++q)
+            {
+                s_gv[threadIdx.x * kQ + q] = make_float4(gv[4 * q], gv[4 * q + 1], gv[4 * q + 2], gv[4 * q + 3]);
+                any |= gv[4 * q] != 0.f || gv[4 * q + 1] != 0.f || gv[4 * q + 2] != 0.f || gv[4 * q + 3] != 0.f;
+            }
+            has = has && any;
             for (int side = 0; side < 2; ++side)
             {
-                if (l == 0) s_n[wave] = 0;
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                if (has)
-                {
-                    const TriLocal& t  = side ? to : ta;
-                    const int64_t base = (side ? so : sa) * g.s0 + ch0;
+                s_base[threadIdx.x] = (side ? so : sa) * g.s0;
+                const TriLocal& t = side ? to : ta;
+                int32_t n         = 0;
 #pragma unroll
-                    for (int k = 0; k < 8; ++k)
+                for (int k = 0; k < 8; ++k)
+                {
+                    const bool put       = has && t.w[k] != 0.f;
+                    const uint64_t lanes = __ballot(put);
+                    if (put)
                     {
-                        if (t.w[k] == 0.f) continue;
-                        const int32_t e = atomicAdd(&s_n[wave], 1);
-                        s_off[wave][e]  = base + t.off[k];
+                        const int32_t e = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(lanes >> 32),
+                                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)lanes, 0));
+                        s_off[wave][e]  = ch0 + t.off[k];
                         s_w[wave][e]    = make_float2(side ? -t.w[k] : t.w[k], __int_as_float(threadIdx.x));
                     }
+                    n += __popcll(lanes);
                 }
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                const int32_t n = s_n[wave];
-                for (int32_t e = l >> 2; e < n; e += 16)
+                for (int32_t e = l / kCh; e < n; e += 64 / kCh)
                 {
                     const float2 w = s_w[wave][e];
-                    const float v  = reinterpret_cast<const float*>(&s_gv[__float_as_int(w.y)])[l & 3];
-                    if (v != 0.f) atomicAdd(grad_grid + s_off[wave][e] + (l & 3), w.x * v);
+                    const float v  = reinterpret_cast<const float*>(&s_gv[__float_as_int(w.y) * kQ])[l % kCh];
+                    if (v != 0.f) atomicAdd(grad_grid + s_base[__float_as_int(w.y)] + s_off[wave][e] + l % kCh, w.x * v);
                 }
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             }
@@ -350,12 +369,12 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
         {
             int64_t sa, so;
             TriLocal ta, to;
-            float gv[4];
+            float gv[kCh];
             int32_t ch0;
             if (!eval(i, sa, so, ta, to, gv, ch0)) continue;
             if constexpr (kGrad)
             {
-                const int nch = min(4, g.C - ch0);
+                const int nch = min(kCh, g.C - ch0);
                 float* da = grad_grid + sa * g.s0;
                 float* dq = grad_grid + so * g.s0;
 #pragma unroll
@@ -375,11 +394,11 @@ __global__ void __launch_bounds__(kRedThreads) k_edge_direct(GridArgs g, const f
 }
 
 // loss = sum(partials) * weight / P with P = row[num_candidates] read on the device (0 when there are no pairs)
-__global__ void __launch_bounds__(kRedThreads) k_sum_partials_per_pair(const double* partials, int64_t n,
+__global__ void __launch_bounds__(kSumThreads) k_sum_partials_per_pair(const double* partials, int64_t n,
                                                                        const int64_t* row, int64_t num_candidates,
                                                                        double weight, double* out)
 {
-    const double t  = block_total(thread_share(partials, n));
+    const double t  = block_total<kSumThreads>(thread_share(partials, n));
     const int64_t P = row[num_candidates];
     if (threadIdx.x == 0) *out = P > 0 ? t * weight / (double)P : 0.0;
 }
@@ -503,13 +522,19 @@ __global__ void __launch_bounds__(kRedThreads) k_tv_fwd(const float* __restrict_
 // thread's entries are issued before any arithmetic, so a wave keeps 7 * kTvPerThread loads in flight; a missing
 // neighbour (at the grid's border) reads the entry itself, whose difference 0 adds nothing to either sum. kDense: the
 // entry's offset within its slot is its index (32-bit offsets).
-template <bool kOverwrite, bool kDense, bool kLoss = true>
+// kV: the entries of an item. 4 takes whole channel quads of a dense channels-last grid (D then counts quads: its C and
+// per_node are divided by 4) in 16-byte loads, so an item's index is split once for four entries: bound by instruction
+// issue otherwise. 4096 grids of 17^3 x 8, overwriting: 409 us entry by entry, 350 us by quads.
+template <bool kOverwrite, bool kDense, bool kLoss = true, int kV = 1>
 __global__ void __launch_bounds__(kRedThreads) k_tv_fwd_bwd(const float* __restrict__ grid, TvDims D, Strides5 S,
                                                             const int64_t* __restrict__ slots, double scale,
                                                             const float* __restrict__ grad_loss,
                                                             float* __restrict__ grad_grid, double* __restrict__ partials)
 {
+    static_assert(kV == 1 || kDense, "quads need a dense grid");
     using Off = typename std::conditional<kDense, int32_t, int64_t>::type;
+    using Vec = typename std::conditional<kV == 4, float4, float>::type;
+    constexpr int kItems = kTvPerThread / kV;
     const int64_t* st = S.s;
     const uint32_t L  = xcd_block(blockIdx.x, gridDim.x);
     if (L >= D.blocks)
@@ -518,7 +543,7 @@ __global__ void __launch_bounds__(kRedThreads) k_tv_fwd_bwd(const float* __restr
         return;
     }
     const int64_t a  = L / D.blocks_per_node;
-    const int32_t e0 = (int32_t)(L - a * D.blocks_per_node) * (kRedThreads * kTvPerThread) + threadIdx.x;
+    const int32_t e0 = (int32_t)(L - a * D.blocks_per_node) * (kRedThreads * kItems) + threadIdx.x;
     const int64_t sl = slots[a];
     if (sl < 0 || sl >= D.N)
     {
@@ -530,46 +555,65 @@ __global__ void __launch_bounds__(kRedThreads) k_tv_fwd_bwd(const float* __restr
     float* d0        = grad_grid + b0;
     const int32_t G  = D.G;
     const Off sx = (Off)st[4], sy = (Off)st[3], sz = (Off)st[2];
-    Off off[kTvPerThread];
-    float v[kTvPerThread][7];  // the entry, its +x +y +z and -x -y -z neighbours
+    Off off[kItems];
+    Vec v[kItems][7];  // the item, its +x +y +z and -x -y -z neighbours
+    auto at = [&](Off o) { return *reinterpret_cast<const Vec*>(g0 + o); };
 #pragma unroll
-    for (int k = 0; k < kTvPerThread; ++k)
+    for (int k = 0; k < kItems; ++k)
     {
         const int32_t e = min(e0 + k * kRedThreads, D.per_node - 1);
         const TvEntry t = tv_entry(e, D);
-        const Off o = kDense ? (Off)e : (Off)(t.c * st[1] + t.z * st[2] + t.y * st[3] + t.x * st[4]);
+        const Off o = kDense ? (Off)e * kV : (Off)(t.c * st[1] + t.z * st[2] + t.y * st[3] + t.x * st[4]);
         off[k]      = o;
-        v[k][0]     = g0[o];
-        v[k][1]     = g0[o + (t.x + 1 < G ? sx : 0)];
-        v[k][2]     = g0[o + (t.y + 1 < G ? sy : 0)];
-        v[k][3]     = g0[o + (t.z + 1 < G ? sz : 0)];
-        v[k][4]     = g0[o - (t.x > 0 ? sx : 0)];
-        v[k][5]     = g0[o - (t.y > 0 ? sy : 0)];
-        v[k][6]     = g0[o - (t.z > 0 ? sz : 0)];
+        v[k][0]     = at(o);
+        v[k][1]     = at(o + (t.x + 1 < G ? sx : 0));
+        v[k][2]     = at(o + (t.y + 1 < G ? sy : 0));
+        v[k][3]     = at(o + (t.z + 1 < G ? sz : 0));
+        v[k][4]     = at(o - (t.x > 0 ? sx : 0));
+        v[k][5]     = at(o - (t.y > 0 ? sy : 0));
+        v[k][6]     = at(o - (t.z > 0 ? sz : 0));
     }
     const double gs = (double)*grad_loss * scale;
     double sum      = 0.0;
 #pragma unroll
-    for (int k = 0; k < kTvPerThread; ++k)
+    for (int k = 0; k < kItems; ++k)
     {
         if (e0 + k * kRedThreads >= D.per_node) break;
-        const float v0 = v[k][0];
-        float acc = 0.f, s = 0.f;
+        float gv[kV];
 #pragma unroll
-        for (int j = 1; j <= 3; ++j)
+        for (int q = 0; q < kV; ++q)
         {
-            const float d = v[k][j] - v0;
-            acc += fabsf(d);
-            s -= sgn(d);
-        }
+            auto comp      = [&](int j) { return reinterpret_cast<const float*>(&v[k][j])[q]; };
+            const float v0 = comp(0);
+            float acc      = 0.f;
+            // -sign(next - v) and sign(v - prev) are both [v > other] - [v < other]: counted as whole numbers
+            int32_t s = 0;
 #pragma unroll
-        for (int j = 4; j <= 6; ++j) s += sgn(v0 - v[k][j]);
-        sum += (double)acc;
-        const float gv = (float)(gs * s);
-        if constexpr (kOverwrite)
-            d0[off[k]] = gv;
+            for (int j = 1; j <= 6; ++j)
+            {
+                const float o = comp(j);
+                if (j <= 3) acc += fabsf(o - v0);
+                s += v0 > o;
+                s -= v0 < o;
+            }
+            sum += (double)acc;
+            gv[q] = (float)(gs * (double)s);
+        }
+        Vec* dst = reinterpret_cast<Vec*>(d0 + off[k]);
+        if constexpr (kV == 4)
+        {
+            float4 g = make_float4(gv[0], gv[1], gv[2], gv[3]);
+            if constexpr (!kOverwrite)
+            {
+                const float4 p = *dst;
+                g.x += p.x, g.y += p.y, g.z += p.z, g.w += p.w;
+            }
+            *dst = g;
+        }
+        else if constexpr (kOverwrite)
+            *dst = gv[0];
         else
-            d0[off[k]] += gv;
+            *dst += gv[0];
     }
     if constexpr (kLoss)
     {
@@ -607,6 +651,32 @@ static TvDims tv_dims(int32_t C, int32_t G, const int64_t* strides, int entries_
     return D;
 }
 
+// the combined pass over the active grids; returns the number of loss partials
+template <bool kOverwrite, bool kLoss>
+static int64_t launch_tv_fwd_bwd(hipStream_t s, const float* grid, int64_t N, int32_t C, int32_t G,
+                                 const int64_t* strides, const int64_t* slots, int64_t num_active, double scale,
+                                 const float* grad_loss, float* grad_grid, double* part)
+{
+    TvDims D          = tv_dims(C, G, strides, kRedThreads * kTvPerThread, num_active, N);
+    const int64_t nb  = xcd_grid(D.blocks);
+    const Strides5 S5 = strides5(strides);
+    // whole channel quads, 16-byte aligned: a block's 2048 entries are 512 quads, so the partials stay as they are
+    if (D.dense && D.channels_last && C % 4 == 0 && strides[0] % 4 == 0 && reinterpret_cast<uintptr_t>(grid) % 16 == 0 &&
+        reinterpret_cast<uintptr_t>(grad_grid) % 16 == 0)
+    {
+        D = tv_dims(C / 4, G, strides, kRedThreads * kTvPerThread / 4, num_active, N);
+        k_tv_fwd_bwd<kOverwrite, true, kLoss, 4><<<(unsigned)nb, kRedThreads, 0, s>>>(grid, D, S5, slots, scale,
+                                                                                     grad_loss, grad_grid, part);
+    }
+    else if (D.dense)
+        k_tv_fwd_bwd<kOverwrite, true, kLoss><<<(unsigned)nb, kRedThreads, 0, s>>>(grid, D, S5, slots, scale, grad_loss,
+                                                                                  grad_grid, part);
+    else
+        k_tv_fwd_bwd<kOverwrite, false, kLoss><<<(unsigned)nb, kRedThreads, 0, s>>>(grid, D, S5, slots, scale, grad_loss,
+                                                                                   grad_grid, part);
+    return nb;
+}
+
 static void launch_candidates(hipStream_t s, const float* pmin, const float* pmax, const uint8_t* flags,
                               int32_t num_nodes, const int64_t* ids, int64_t n, int32_t G, float eps, int32_t* other,
                               int64_t* is_pair)
@@ -621,20 +691,20 @@ static void launch_candidates(hipStream_t s, const float* pmin, const float* pma
                                                            is_pair);
 }
 
-template <typename I, bool V>
+template <typename I, bool V, int Q>
 static void launch_edge_direct(unsigned nb, hipStream_t s, bool want_loss, bool want_grad, const GridArgs& g,
                                const float* pmin, const float* pmax, const int64_t* ids, const int64_t* slot,
                                int64_t n, int32_t G, const int32_t* other, const int64_t* row, uint64_t seed,
                                double weight, const float* gl, float* gg, double* part)
 {
     if (want_loss && want_grad)
-        k_edge_direct<I, V, true, true><<<nb, kRedThreads, 0, s>>>(g, pmin, pmax, ids, slot, n, G, other, row, seed,
+        k_edge_direct<I, V, Q, true, true><<<nb, kRedThreads, 0, s>>>(g, pmin, pmax, ids, slot, n, G, other, row, seed,
                                                                    weight, gl, gg, part);
     else if (want_loss)
-        k_edge_direct<I, V, true, false><<<nb, kRedThreads, 0, s>>>(g, pmin, pmax, ids, slot, n, G, other, row, seed,
+        k_edge_direct<I, V, Q, true, false><<<nb, kRedThreads, 0, s>>>(g, pmin, pmax, ids, slot, n, G, other, row, seed,
                                                                     weight, nullptr, nullptr, part);
     else
-        k_edge_direct<I, V, false, true><<<nb, kRedThreads, 0, s>>>(g, pmin, pmax, ids, slot, n, G, other, row, seed,
+        k_edge_direct<I, V, Q, false, true><<<nb, kRedThreads, 0, s>>>(g, pmin, pmax, ids, slot, n, G, other, row, seed,
                                                                     weight, gl, gg, part);
 }
 
@@ -714,7 +784,7 @@ extern "C"
         k_edge_fwd<<<(unsigned)nb, kRedThreads, 0, s>>>(features, num_pairs, C, seed, part);
         NEAT_LAUNCHED();
         // loss = mean_p(edge_error_p) * weight * C
-        k_sum_partials<<<1, kRedThreads, 0, s>>>(part, nb, weight * C / (double)num_pairs, loss);
+        k_sum_partials<<<1, kSumThreads, 0, s>>>(part, nb, weight * C / (double)num_pairs, loss);
         NEAT_LAUNCHED();
         return NEAT_OK;
     }
@@ -756,7 +826,7 @@ extern "C"
         k_tv_fwd<<<(unsigned)nb, kRedThreads, 0, s>>>(grid, D, strides5(strides), slots, part);
         NEAT_LAUNCHED();
         // each axis: mean over (A, C, G, G, G - 1) differences; the three axes have equal counts; times C * weight
-        k_sum_partials<<<1, kRedThreads, 0, s>>>(part, nb, weight * C / ((double)num_active * C * G * G * (G - 1)),
+        k_sum_partials<<<1, kSumThreads, 0, s>>>(part, nb, weight * C / ((double)num_active * C * G * G * (G - 1)),
                                                  loss);
         NEAT_LAUNCHED();
         return NEAT_OK;
@@ -773,15 +843,10 @@ extern "C"
                      (long long)N);
         NEAT_REQUIRE(C * (int64_t)G * G * G < (1 << 24) && C < 256 && G < 256,
                      "neat_tv_loss_bwd: C * G^3 must be below 2^24, C and G below 256");
-        const TvDims D     = tv_dims(C, G, strides, kRedThreads * kTvPerThread, num_active, N);
         const double scale = weight * C / ((double)num_active * C * G * G * (G - 1));
         // the combined pass without its loss: same per-entry gradient, all of a thread's loads issued first
-        if (D.dense)
-            k_tv_fwd_bwd<false, true, false><<<(unsigned)xcd_grid(D.blocks), kRedThreads, 0, as_stream(stream)>>>(
-                grid, D, strides5(strides), slots, scale, grad_loss, grad_grid, nullptr);
-        else
-            k_tv_fwd_bwd<false, false, false><<<(unsigned)xcd_grid(D.blocks), kRedThreads, 0, as_stream(stream)>>>(
-                grid, D, strides5(strides), slots, scale, grad_loss, grad_grid, nullptr);
+        launch_tv_fwd_bwd<false, false>(as_stream(stream), grid, N, C, G, strides, slots, num_active, scale, grad_loss,
+                                        grad_grid, nullptr);
         NEAT_LAUNCHED();
         return NEAT_OK;
     }
@@ -806,25 +871,14 @@ extern "C"
                      "neat_tv_loss_fwd_bwd: C * G^3 must be below 2^24, C and G below 256");
         NEAT_REQUIRE(workspace && workspace_bytes >= neat_tv_workspace_bytes(num_active, C, G),
                      "neat_tv_loss_fwd_bwd: workspace too small");
-        const TvDims D     = tv_dims(C, G, strides, kRedThreads * kTvPerThread, num_active, N);
-        const int64_t nb   = xcd_grid(D.blocks);
         const double scale = weight * C / ((double)num_active * C * G * G * (G - 1));
         double* part       = static_cast<double*>(workspace);
-        const Strides5 S5 = strides5(strides);
-        if (overwrite && D.dense)
-            k_tv_fwd_bwd<true, true><<<(unsigned)nb, kRedThreads, 0, s>>>(grid, D, S5, slots, scale, grad_loss, grad_grid,
-                                                                           part);
-        else if (overwrite)
-            k_tv_fwd_bwd<true, false><<<(unsigned)nb, kRedThreads, 0, s>>>(grid, D, S5, slots, scale, grad_loss,
-                                                                            grad_grid, part);
-        else if (D.dense)
-            k_tv_fwd_bwd<false, true><<<(unsigned)nb, kRedThreads, 0, s>>>(grid, D, S5, slots, scale, grad_loss,
-                                                                            grad_grid, part);
-        else
-            k_tv_fwd_bwd<false, false><<<(unsigned)nb, kRedThreads, 0, s>>>(grid, D, S5, slots, scale, grad_loss,
-                                                                             grad_grid, part);
+        const int64_t nb   = overwrite ? launch_tv_fwd_bwd<true, true>(s, grid, N, C, G, strides, slots, num_active, scale,
+                                                                       grad_loss, grad_grid, part)
+                                       : launch_tv_fwd_bwd<false, true>(s, grid, N, C, G, strides, slots, num_active,
+                                                                        scale, grad_loss, grad_grid, part);
         NEAT_LAUNCHED();
-        k_sum_partials<<<1, kRedThreads, 0, s>>>(part, nb, scale, loss);
+        k_sum_partials<<<1, kSumThreads, 0, s>>>(part, nb, scale, loss);
         NEAT_LAUNCHED();
         return NEAT_OK;
     }
@@ -873,29 +927,34 @@ extern "C"
         int st = exclusive_scan_i64(s, row, n, scan_ws, scan_bytes);  // row[n] = number of pairs P
         if (st) return st;
         GridArgs g{grid, strides[0], strides[1], strides[2], strides[3], strides[4], N, C, G, G, G};
-        const int64_t total = n * ((C + 3) / 4);  // lanes: (candidate, channel quad)
-        const unsigned nb   = (unsigned)std::min<int64_t>(blocks_for(total, kRedThreads), kEdgeDirectBlocks);
         // 16-byte loads: channels contiguous, whole quads, every corner offset a multiple of 4 floats
         const bool vec4 = strides[1] == 1 && C % 4 == 0 && strides[0] % 4 == 0 && strides[2] % 4 == 0 &&
                           strides[3] % 4 == 0 && strides[4] % 4 == 0 && reinterpret_cast<uintptr_t>(grid) % 16 == 0;
-        const bool small = total < ((int64_t)1 << 31);
+        // a lane's channels: two quads where they are whole (the pair's geometry is then worked out once for both)
+        const int quads     = vec4 && C % 8 == 0 ? 2 : 1;
+        const int64_t total = n * ((C + 4 * quads - 1) / (4 * quads));  // lanes
+        const unsigned nb   = (unsigned)std::min<int64_t>(blocks_for(total, kRedThreads), kEdgeDirectBlocks);
+        const bool small    = total < ((int64_t)1 << 31);
         const bool wl = loss != nullptr, wg = grad_grid != nullptr;
-        if (small && vec4)
-            launch_edge_direct<uint32_t, true>(nb, s, wl, wg, g, node_pos_min, node_pos_max, active_node_ids, node_slot,
-                                               n, G, other, row, seed, weight, grad_loss, grad_grid, part);
-        else if (small)
-            launch_edge_direct<uint32_t, false>(nb, s, wl, wg, g, node_pos_min, node_pos_max, active_node_ids,
-                                                node_slot, n, G, other, row, seed, weight, grad_loss, grad_grid, part);
+        auto launch = [&](auto idx, auto v, auto q)
+        {
+            launch_edge_direct<decltype(idx), decltype(v)::value, decltype(q)::value>(
+                nb, s, wl, wg, g, node_pos_min, node_pos_max, active_node_ids, node_slot, n, G, other, row, seed, weight,
+                grad_loss, grad_grid, part);
+        };
+        auto by_index = [&](auto v, auto q) { small ? launch(uint32_t{}, v, q) : launch(int64_t{}, v, q); };
+        using One = std::integral_constant<int, 1>;
+        using Two = std::integral_constant<int, 2>;
+        if (quads == 2)
+            by_index(std::true_type{}, Two{});
         else if (vec4)
-            launch_edge_direct<int64_t, true>(nb, s, wl, wg, g, node_pos_min, node_pos_max, active_node_ids, node_slot,
-                                              n, G, other, row, seed, weight, grad_loss, grad_grid, part);
+            by_index(std::true_type{}, One{});
         else
-            launch_edge_direct<int64_t, false>(nb, s, wl, wg, g, node_pos_min, node_pos_max, active_node_ids, node_slot,
-                                               n, G, other, row, seed, weight, grad_loss, grad_grid, part);
+            by_index(std::false_type{}, One{});
         NEAT_LAUNCHED();
         if (loss)
         {
-            k_sum_partials_per_pair<<<1, kRedThreads, 0, s>>>(part, nb, row, n, weight, loss);
+            k_sum_partials_per_pair<<<1, kSumThreads, 0, s>>>(part, nb, row, n, weight, loss);
             NEAT_LAUNCHED();
         }
         return NEAT_OK;
