@@ -936,7 +936,7 @@ int fwd_workgroups(const ProjSizes& z) { return (int)std::max<int64_t>(1, std::m
 size_t partials_bytes(const ProjSizes& z)
 {
     size_t slices = std::max<size_t>({(size_t)bw1_workgroups(z), (size_t)bf16_bwd_slices(mfma_bwd_workgroups(z)),
-                                      (size_t)kNodeWGMax * kNodeWaves});
+                                      (size_t)kNodeWGMax});
     return (slices * z.P * 4 + 255) / 256 * 256;
 }
 
@@ -1182,7 +1182,7 @@ int launch_bw_mfma(hipStream_t s, const Args& a, const Plan& p, const BwdBufs& b
     const bool relu16 = P::kBF16 && a.relu16;
     const bool relu32 = !P::kBF16 && a.act == NEAT_ACT_RELU;
     const int nwg     = mfma_bwd_workgroups(a.z);
-    const int slices  = relu16 ? p.nwg * kNodeWaves : (P::kBF16 ? bf16_bwd_slices(nwg) : (relu32 ? nwg : nwg * 4));
+    const int slices  = relu16 ? p.nwg : (P::kBF16 ? bf16_bwd_slices(nwg) : (relu32 ? nwg : nwg * 4));
     const int Ptot    = a.m.nparams();
     if (stage == 1)
     {

@@ -675,9 +675,9 @@ __device__ __forceinline__ void stage_node_grid(const uint4* __restrict__ src, u
 int launch_mfma_fwd_relu(hipStream_t s, int H, const ProjGeom& g, const Plan& p, const float* params,
                          const void* grid_bf16, float* seg_partial, float* sample_out);
 
-// Launches k_mfma_bwd_relu<H> (H = 32 or 64) on the plan's p.nwg node-resident workgroups of kNodeThreads; every
-// wave writes one parameter-gradient slice (p.nwg * kNodeWaves slices). It reads the per-sample caches that
-// k_mfma_fwd_relu wrote into the same plan: the forward must have run on it with the same arguments.
+// Launches k_mfma_bwd_relu<H> (H = 32 or 64) on the plan's p.nwg node-resident workgroups of kNodeThreads, each
+// of which writes one parameter-gradient slice (p.nwg slices). It reads the per-sample caches that k_mfma_fwd_relu
+// wrote into the same plan: the forward must have run on it with the same arguments.
 int launch_mfma_bwd_relu(hipStream_t s, int H, const ProjGeom& g, const Plan& p, const float* params,
                          const float* grad_proj, float* dfeat, unsigned int* dmax, float* partials, int32_t P_total);
 

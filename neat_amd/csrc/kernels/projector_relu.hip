@@ -113,6 +113,8 @@ __global__ void __launch_bounds__(kNodeThreads, 2) k_mfma_bwd_relu(ProjGeom g, P
     __shared__ ChunkCtx cx;
     __shared__ __align__(16) float s_dz[kNodeWaves][32];
     __shared__ __align__(16) unsigned short s_tr[kNodeWaves][32 * kTrRow];
+    constexpr int kParams = H * C + H + H * H + H + H + 1, kRedSlices = 4;
+    __shared__ float s_red[kRedSlices][kParams];
     load_weights_relu<H>(params, w);
     __syncthreads();  // the final partial write reads w.w3 even in a workgroup that gets no chunk
     const int l = threadIdx.x & 63, wave = threadIdx.x >> 6, n = l & 31, hg = l >> 5;
@@ -331,29 +333,45 @@ __global__ void __launch_bounds__(kNodeThreads, 2) k_mfma_bwd_relu(ProjGeom g, P
         if (l == 0) atomicMax(dmax + 1 + slot, __float_as_uint(cmax));
         amax = fmaxf(amax, cmax);
     }
-    // ---- this wave's slice of the partial parameter gradient (packed layout); rows scaled by the output weights
-    // where the output weights were folded out of D2 ----
-    float* part   = partials + ((int64_t)blockIdx.x * kNodeWaves + wave) * P_total;
+    // ---- the workgroup's slice of the partial parameter gradient (packed layout): its waves' sums added in a fixed
+    // order in LDS, kRedSlices waves at a time; rows scaled by the output weights where those were folded out of D2 ----
     const int oW0 = 0, ob0 = H * C, oW1 = ob0 + H, ob1 = oW1 + H * H, oW2 = ob1 + H, ob2 = oW2 + H;
 #pragma unroll
-    for (int m2 = 0; m2 < MT; ++m2)
-    {
-#pragma unroll
-        for (int i2 = 0; i2 < 16; ++i2)
-        {
-            const int r    = 32 * m2 + crow(i2, hg);
-            const float s3 = w.w3[r];
-#pragma unroll
-            for (int m1 = 0; m1 < MT; ++m1) part[oW1 + r * H + 32 * m1 + n] = dW2[m2][m1][i2] * s3;
-            if (n < C) part[oW0 + r * C + n] = E[m2][i2];
-            if (n == 8) part[ob0 + r] = E[m2][i2];
-            if (n == 9) part[oW2 + r] = E[m2][i2];
-            if (n == 10) part[ob1 + r] = E[m2][i2] * s3;
-        }
-    }
-#pragma unroll
     for (int off = 16; off >= 1; off >>= 1) b3 += __shfl_xor(b3, off);
-    if (l == 0) part[ob2] = b3;
+    for (int k = 0; k < kNodeWaves; k += kRedSlices)
+    {
+        if (wave >= k && wave < k + kRedSlices)
+        {
+            float* red = s_red[wave - k];
+            auto put   = [&](int i, float v) { red[i] = k > 0 ? red[i] + v : v; };
+#pragma unroll
+            for (int m2 = 0; m2 < MT; ++m2)
+            {
+#pragma unroll
+                for (int i2 = 0; i2 < 16; ++i2)
+                {
+                    const int r    = 32 * m2 + crow(i2, hg);
+                    const float s3 = w.w3[r];
+#pragma unroll
+                    for (int m1 = 0; m1 < MT; ++m1) put(oW1 + r * H + 32 * m1 + n, dW2[m2][m1][i2] * s3);
+                    if (n < C) put(oW0 + r * C + n, E[m2][i2]);
+                    if (n == 8) put(ob0 + r, E[m2][i2]);
+                    if (n == 9) put(oW2 + r, E[m2][i2]);
+                    if (n == 10) put(ob1 + r, E[m2][i2] * s3);
+                }
+            }
+            if (l == 0) put(ob2, b3);
+        }
+        __syncthreads();
+    }
+    float* part = partials + (int64_t)blockIdx.x * P_total;
+    for (int t = threadIdx.x; t < kParams; t += kNodeThreads)
+    {
+        float v = s_red[0][t];
+#pragma unroll
+        for (int k = 1; k < kRedSlices; ++k) v += s_red[k][t];
+        part[t] = v;
+    }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
     if (l == 0) atomicMax(dmax, __float_as_uint(amax));
