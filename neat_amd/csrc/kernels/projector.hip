@@ -25,14 +25,119 @@ namespace neat
 {
 
 // ---- plan ---------------------------------------------------------------------------------------------------------
+// a segment's sort key: its node's slot; invalid slots sort last
+__device__ __forceinline__ int32_t plan_key(const ProjGeom& g, int64_t k)
+{
+    const int32_t node = g.seg_node[k];
+    const int64_t slot = (node >= 0 && node < g.num_nodes) ? g.prefix[node] : -1;
+    return (slot >= 0 && slot < g.N) ? (int32_t)slot : (int32_t)g.N;
+}
+
 __global__ void __launch_bounds__(256) k_plan_keys(ProjGeom g, int32_t* keys, int32_t* vals)
 {
     int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= g.K) return;
-    int32_t node = g.seg_node[k];
-    int64_t slot = (node >= 0 && node < g.num_nodes) ? g.prefix[node] : -1;
-    keys[k]      = (slot >= 0 && slot < g.N) ? (int32_t)slot : (int32_t)g.N;  // invalid slots sort last
-    vals[k]      = (int32_t)k;
+    keys[k] = plan_key(g, k);
+    vals[k] = (int32_t)k;
+}
+
+// The segments' stable sort by slot as counting sorts by digits of at most 8 bits, least first: a tile per workgroup
+// counts its digits (k_sort_count, counts digit-major so that one scan gives every tile's first place per digit) and
+// then places its items (k_sort_place). A wave takes 64 consecutive items at a time: the lanes of equal digit find
+// each other by ballots, an item's place is its tile's first place of the digit, plus the items of the digit in the
+// tile's earlier waves, in its wave's earlier rounds and in lower lanes. The first digit's passes compute the keys.
+// Up to about a million segments bound by launches and their gaps (6, or 3 with one digit): 4096 slots, 400,000
+// segments: the plan 177 us with the library's sort (a merge sort of 21 launches), 127 us like this.
+constexpr int kSortThreads = 512, kSortWaves = kSortThreads / 64;
+constexpr int kSortRounds  = 4, kSortTile = kSortThreads * kSortRounds, kSortBins = 256;
+
+template <bool kFirst>
+__global__ void __launch_bounds__(kSortThreads) k_sort_count(ProjGeom g, int32_t* keys, int64_t* counts, int shift,
+                                                             int bins)
+{
+    __shared__ int32_t cnt[kSortBins];
+    if (threadIdx.x < bins) cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t k0 = (int64_t)blockIdx.x * kSortTile + threadIdx.x;
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r)
+    {
+        const int64_t k = k0 + r * kSortThreads;
+        if (k >= g.K) break;
+        int32_t key;
+        if constexpr (kFirst)
+        {
+            key     = plan_key(g, k);
+            keys[k] = key;
+        }
+        else
+            key = keys[k];
+        atomicAdd(&cnt[(key >> shift) & (bins - 1)], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < bins) counts[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = cnt[threadIdx.x];
+}
+
+// counts: scanned. vals null: an item's value is its index.
+__global__ void __launch_bounds__(kSortThreads) k_sort_place(const int32_t* __restrict__ keys,
+                                                             const int32_t* __restrict__ vals, int64_t K,
+                                                             const int64_t* __restrict__ counts, int shift, int bins,
+                                                             int32_t* __restrict__ out_keys,
+                                                             int32_t* __restrict__ out_vals)
+{
+    __shared__ int32_t cnt[kSortWaves][kSortBins];
+    for (int i = threadIdx.x; i < kSortWaves * kSortBins; i += kSortThreads) (&cnt[0][0])[i] = 0;
+    __syncthreads();
+    const int l = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t k0 = (int64_t)blockIdx.x * kSortTile + wave * (64 * kSortRounds) + l;
+    int32_t key[kSortRounds], val[kSortRounds], place[kSortRounds];
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r)
+    {
+        const int64_t k = k0 + 64 * r;
+        key[r]          = k < K ? keys[k] : 0;
+        val[r]          = k < K && vals ? vals[k] : (int32_t)k;
+    }
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r)
+    {
+        const bool in    = k0 + 64 * r < K;
+        const int32_t d  = (key[r] >> shift) & (bins - 1);
+        uint64_t same    = __ballot(in);
+        for (int bit = 1; bit < bins; bit <<= 1)
+        {
+            const uint64_t set = __ballot((d & bit) != 0);
+            same &= (d & bit) ? set : ~set;
+        }
+        const uint32_t before = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0));
+        const int32_t had = cnt[wave][d];
+        place[r]          = had + (int32_t)before;
+        wave_lds_fence();
+        if (in && before == 0) cnt[wave][d] = had + __popcll(same);
+        wave_lds_fence();
+    }
+    __syncthreads();
+    if (threadIdx.x < bins)
+    {
+        int32_t at = (int32_t)counts[(int64_t)threadIdx.x * gridDim.x + blockIdx.x];
+#pragma unroll
+        for (int w = 0; w < kSortWaves; ++w)
+        {
+            const int32_t n     = cnt[w][threadIdx.x];
+            cnt[w][threadIdx.x] = at;
+            at += n;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r)
+    {
+        if (k0 + 64 * r >= K) break;
+        const int32_t at = cnt[wave][(key[r] >> shift) & (bins - 1)] + place[r];
+        out_keys[at]     = key[r];
+        out_vals[at]     = val[r];
+    }
 }
 
 // First position of the sorted keys in [lo, K) with key >= s.
@@ -877,11 +982,56 @@ int32_t scatter_chunk(int64_t S)
     return (int32_t)std::max<int64_t>(2048, std::min<int64_t>(65536, t));
 }
 
+// bits of the sort keys 0 .. N
+int key_bits(int64_t N)
+{
+    int bits = 1;
+    while (((int64_t)1 << bits) <= N) ++bits;
+    return bits;
+}
+
+// Counting sorts (k_sort_count / k_sort_place) for one digit, or two; the library's radix sort for more, and where it is
+// the faster one. Whole plans, counting against library: one digit, 64 slots, 3,000 / 400,000 / 12 M segments 36 / 89 /
+// 980 us against 41 / 176 / 1009. Two digits, 4096 slots, 20,000 / 400,000 / 4 M segments 74 / 127 / 455 us against
+// 85 / 177 / 462, but 3,000 (the library sorts up to 4096 in one workgroup) 52 against 48; 30,000 slots, 1.5 M segments
+// 236 against 254, 4 M 519 against 498 (the counts of 256 digits a tile weigh more than its items).
+bool own_sort(int64_t K, int64_t N)
+{
+    const int bits = key_bits(N);
+    return K > 0 && (bits <= 8 || (bits <= 16 && K > 4096 && (bits <= 13 || K <= ((int64_t)1 << 21))));
+}
+
+struct SortShape
+{
+    int64_t tiles;
+    int digits, bits, bins;  // digits of `bits` bits each
+};
+
+SortShape sort_shape(int64_t K, int64_t N)
+{
+    SortShape q;
+    const int bits = key_bits(N);
+    q.tiles        = (K + kSortTile - 1) / kSortTile;
+    q.digits       = bits <= 8 ? 1 : 2;
+    q.bits         = (bits + q.digits - 1) / q.digits;
+    q.bins         = 1 << q.bits;
+    return q;
+}
+
+size_t sort_items_bytes(int64_t K) { return (4 * (size_t)K + 255) / 256 * 256; }
+size_t sort_counts_bytes(const SortShape& q) { return (8 * (size_t)(q.tiles * q.bins + 1) + 255) / 256 * 256; }
+
 ProjSizes proj_sizes(int64_t K, int64_t S, int64_t N, int32_t G, int32_t C, int32_t P, bool prop)
 {
     ProjSizes z{K, S, N, G, C, P, 0, 0, scatter_chunk(S), 0, prop};
     z.max1 = (S + (int64_t)kSegCost * K + kFwdChunk - 1) / kFwdChunk + N;
     z.max2 = (S + z.chunk2 - 1) / z.chunk2 + N;
+    if (own_sort(K, N))
+    {
+        const SortShape q = sort_shape(K, N);
+        z.sort_temp       = 2 * sort_items_bytes(K) + sort_counts_bytes(q) + scan_workspace_bytes(q.tiles * q.bins + 1);
+        return z;
+    }
     size_t tmp = 0;
     hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, (int32_t*)nullptr, (int32_t*)nullptr, (int32_t*)nullptr,
                                        (int32_t*)nullptr, (int)std::max<int64_t>(K, 1), 0, 32);
@@ -1533,13 +1683,40 @@ extern "C"
         size_t temp_sz  = proj_layout(z).off[11] - proj_layout(z).off[10];
         if (z.K > 0)
         {
-            k_plan_keys<<<grid_for(z.K, 256), 256, 0, s>>>(a.g, keys, vals);
-            NEAT_LAUNCHED();
-            int end_bit = 1;
-            while (((int64_t)1 << end_bit) <= z.N) ++end_bit;
-            size_t tmp = z.sort_temp;
-            NEAT_HIP(hipcub::DeviceRadixSort::SortPairs(temp, tmp, keys, skeys, vals, p.perm, (int)z.K, 0, end_bit,
-                                                        s));
+            if (own_sort(z.K, z.N))
+            {
+                const SortShape q = sort_shape(z.K, z.N);
+                char* w           = static_cast<char*>(temp);
+                int32_t* mid_keys = reinterpret_cast<int32_t*>(w);
+                int32_t* mid_vals = reinterpret_cast<int32_t*>(w + sort_items_bytes(z.K));
+                int64_t* counts   = reinterpret_cast<int64_t*>(w + 2 * sort_items_bytes(z.K));
+                void* scan_ws     = w + 2 * sort_items_bytes(z.K) + sort_counts_bytes(q);
+                const size_t sb   = scan_workspace_bytes(q.tiles * q.bins + 1);
+                for (int d = 0; d < q.digits; ++d)
+                {
+                    const bool last    = d == q.digits - 1;
+                    int32_t* in_keys   = d == 0 ? keys : mid_keys;
+                    const unsigned nwg = (unsigned)q.tiles;
+                    if (d == 0)
+                        k_sort_count<true><<<nwg, kSortThreads, 0, s>>>(a.g, in_keys, counts, 0, q.bins);
+                    else
+                        k_sort_count<false><<<nwg, kSortThreads, 0, s>>>(a.g, in_keys, counts, d * q.bits, q.bins);
+                    NEAT_LAUNCHED();
+                    if ((st = exclusive_scan_i64(s, counts, q.tiles * q.bins, scan_ws, sb))) return st;
+                    k_sort_place<<<nwg, kSortThreads, 0, s>>>(in_keys, d == 0 ? nullptr : mid_vals, z.K, counts,
+                                                              d * q.bits, q.bins, last ? skeys : mid_keys,
+                                                              last ? p.perm : mid_vals);
+                    NEAT_LAUNCHED();
+                }
+            }
+            else
+            {
+                k_plan_keys<<<grid_for(z.K, 256), 256, 0, s>>>(a.g, keys, vals);
+                NEAT_LAUNCHED();
+                size_t tmp = z.sort_temp;
+                NEAT_HIP(hipcub::DeviceRadixSort::SortPairs(temp, tmp, keys, skeys, vals, p.perm, (int)z.K, 0,
+                                                            key_bits(z.N), s));
+            }
             k_plan_records<<<grid_for(z.K, 256), 256, 0, s>>>(a.g, p, reinterpret_cast<float*>(region(ws, z, 11)));
             NEAT_LAUNCHED();
         }
