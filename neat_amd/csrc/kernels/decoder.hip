@@ -148,12 +148,11 @@ __global__ void __launch_bounds__(256) k_dec_mfma_bwd(const float* __restrict__ 
                                                       float* __restrict__ partials, int32_t P_total)
 {
     typedef PrecF32 P;
-    typedef Stage<P> ST;
     __shared__ WeightLDS<P, H> w;
-    __shared__ __align__(16) typename ST::E stage[kDecMfmaWaves][ST::elems(H)];
+    __shared__ __align__(16) float stage[kDecMfmaWaves][Stage::elems(H)];
     load_weights<P, H, 8>(params, w);
     const int l = threadIdx.x & 63, wave = threadIdx.x >> 6, hg = l >> 5;
-    BwdStage<P, H> sb(stage[wave]);
+    BwdStage<H> sb(stage[wave]);
     BwdAcc<H / 32> acc;
     __syncthreads();
     const int64_t tiles = (S + 31) / 32;
@@ -163,7 +162,7 @@ __global__ void __launch_bounds__(256) k_dec_mfma_bwd(const float* __restrict__ 
         const bool valid = i < S;
         float x4[4];
         load_x4(x, i, S, x4);
-        const f32x16 dx = tile_backward_mfma<P, H, ACT>(w, x4, valid ? gy[i] : 0.f, valid, last_act, beta, sb, acc);
+        const f32x16 dx = tile_backward_mfma<H, ACT>(w, x4, valid ? gy[i] : 0.f, valid, last_act, beta, sb, acc);
         if (gx && valid)
         {
 #pragma unroll

@@ -262,25 +262,16 @@ __device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOM
 
 constexpr int kRS = 36;  // row stride (floats) of the backward's [row][sample] staging buffers (16-byte rows)
 
-// A / B fragment of a weight-gradient product over the tile's 32 samples, from a [row][sample] staging buffer:
-// FP32 step st covers samples 2st + l/32; BF16 step st covers samples 16st + 8(l/32) + j.
-template <typename P>
-__device__ __forceinline__ typename P::Frag stage_frag(const float* buf, int row, int st, int hg, bool zero)
+// BF16 A / B fragment of a weight-gradient product over the tile's 32 samples, from a [row][sample] staging buffer:
+// step st covers samples 16st + 8(l/32) + j. Masked lanes read row 0 (always inside the buffer) and discard it.
+__device__ __forceinline__ bf16x8 stage_frag(const float* buf, int row, int st, int hg, bool zero)
 {
-    typename P::Frag f;
-    if constexpr (P::kBF16)
-    {
-        // masked lanes read row 0 (always inside the buffer) and discard it
-        const float4* src = reinterpret_cast<const float4*>(buf + (zero ? 0 : row) * kRS + 16 * st + 8 * hg);
-        const float4 u = src[0], v = src[1];
-        const float e[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+    const float4* src = reinterpret_cast<const float4*>(buf + (zero ? 0 : row) * kRS + 16 * st + 8 * hg);
+    const float4 u = src[0], v = src[1];
+    const float e[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+    bf16x8 f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = (__bf16)(zero ? 0.f : e[j]);
-    }
-    else
-    {
-        f = zero ? 0.f : buf[row * kRS + 2 * st + hg];
-    }
+    for (int j = 0; j < 8; ++j) f[j] = (__bf16)(zero ? 0.f : e[j]);
     return f;
 }
 
@@ -288,55 +279,33 @@ __device__ __forceinline__ typename P::Frag stage_frag(const float* buf, int row
 // gradients (E = dZ1 [x; 1]^T + dZ2 [e10]^T + h2 [dz e9]^T, with the B operand masked per product).
 constexpr int kXOnes1 = 8, kXDz = 9, kXOnes2 = 10, kXRows = 11;
 
-// The backward's [row][sample] staging buffers: BF16 (rows of 40) for the BF16 form, where the values are rounded
-// once when staged and read as ready operands, FP32 (rows of kRS) otherwise.
-template <typename P>
+// The FP32 backward's [row][sample] staging buffers.
 struct Stage
 {
-    static constexpr int kStride = P::kBF16 ? 40 : kRS;  // elements per row; 16-byte rows either way
-    typedef typename std::conditional<P::kBF16, unsigned short, float>::type E;
     // elements of one wave's buffers for hidden width h: dZ / activations (2h rows) and the X tile
-    static constexpr int elems(int h) { return (2 * h + kXRows) * kStride; }
-    __device__ static __forceinline__ void put(E* b, int row, int col, float v)
+    static constexpr int elems(int h) { return (2 * h + kXRows) * kRS; }
+    __device__ static __forceinline__ void put(float* b, int row, int col, float v) { b[row * kRS + col] = v; }
+    // A / B fragment over the tile's samples: step st covers samples 2st + l/32; masked lanes read row 0 and discard it
+    __device__ static __forceinline__ float frag(const float* b, int row, int st, int hg, bool zero)
     {
-        if constexpr (P::kBF16)
-            b[row * kStride + col] = (unsigned short)bf16_bits(v);
-        else
-            b[row * kStride + col] = v;
-    }
-    // A / B fragment over the tile's samples (see stage_frag); masked lanes read row 0 and discard it
-    __device__ static __forceinline__ typename P::Frag frag(const E* b, int row, int st, int hg, bool zero)
-    {
-        if constexpr (P::kBF16)
-        {
-            const uint4 u = *reinterpret_cast<const uint4*>(b + (zero ? 0 : row) * kStride + 16 * st + 8 * hg);
-            typename P::Frag f;
-            __builtin_memcpy(&f, &u, sizeof(f));
-            if (zero) f = typename P::Frag{};
-            return f;
-        }
-        else
-        {
-            return zero ? 0.f : b[row * kStride + 2 * st + hg];
-        }
+        return zero ? 0.f : b[row * kRS + 2 * st + hg];
     }
 };
 
 // One wave's staging buffers: sA (H rows), sB (H rows), sX (kXRows rows). The constant rows of sX are set here.
-template <typename P, int H>
+template <int H>
 struct BwdStage
 {
-    typedef typename Stage<P>::E E;
-    E* sA;
-    E* sB;
-    E* sX;
-    __device__ explicit BwdStage(E* base) : sA(base), sB(base + H * Stage<P>::kStride), sX(sB + H * Stage<P>::kStride)
+    float* sA;
+    float* sB;
+    float* sX;
+    __device__ explicit BwdStage(float* base) : sA(base), sB(base + H * kRS), sX(sB + H * kRS)
     {
         const int l = threadIdx.x & 63;
         if (l < 32)
         {
-            Stage<P>::put(sX, kXOnes1, l, 1.f);
-            Stage<P>::put(sX, kXOnes2, l, 1.f);
+            Stage::put(sX, kXOnes1, l, 1.f);
+            Stage::put(sX, kXOnes2, l, 1.f);
         }
     }
 };
@@ -361,18 +330,19 @@ struct BwdAcc
     }
 };
 
-// Backward of one tile of 32 samples on a wave: recompute the forward (tile_forward_mfma), take dz = gy *
+// FP32 backward of one tile of 32 samples on a wave: recompute the forward (tile_forward_mfma), take dz = gy *
 // last_act'(z) (0 for invalid lanes), back-propagate on the matrix cores, and add the tile's parameter-gradient
 // products to acc (products over the tile's samples, staged through LDS as [row][sample]). Returns dL/dx in
 // registers 0..3 of each lane (channels 4g..4g+3 of its sample, g = lane / 32).
-template <typename P, int H, int ACT>
-__device__ __forceinline__ f32x16 tile_backward_mfma(const WeightLDS<P, H>& w, const float (&x4)[4], float gy,
-                                                     bool valid, int last_act, float beta, const BwdStage<P, H>& sb,
+template <int H, int ACT>
+__device__ __forceinline__ f32x16 tile_backward_mfma(const WeightLDS<PrecF32, H>& w, const float (&x4)[4], float gy,
+                                                     bool valid, int last_act, float beta, const BwdStage<H>& sb,
                                                      BwdAcc<H / 32>& acc)
 {
+    typedef PrecF32 P;
+    typedef Stage ST;
     constexpr int MT = H / 32, S = steps_per_tile<P>();
-    constexpr int KSTEPS = 32 / (2 * P::KS);  // sample steps of a weight-gradient product (FP32 16, BF16 2)
-    typedef Stage<P> ST;
+    constexpr int KSTEPS = 32 / (2 * P::KS);  // sample steps of a weight-gradient product
     const int l = threadIdx.x & 63, n = l & 31, hg = l >> 5;
     Fwd<MT> f;
     tile_forward_mfma<P, H, ACT>(w, x4, beta, f);

@@ -878,11 +878,10 @@ __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const floa
     constexpr int MT = H / 32, C = 8;
     __shared__ WeightLDS<P, H> w;
     __shared__ ChunkCtx cx;
-    typedef Stage<P> ST;
-    __shared__ __align__(16) typename ST::E stage[4][ST::elems(H)];
+    __shared__ __align__(16) float stage[4][Stage::elems(H)];
     load_weights<P, H, C>(params, w);
     const int l = threadIdx.x & 63, wave = threadIdx.x >> 6, hg = l >> 5;
-    BwdStage<P, H> sb(stage[wave]);
+    BwdStage<H> sb(stage[wave]);
     BwdAcc<MT> acc;
     float amax = 0.f;  // largest |dL/dfeature| this lane wrote
     const int64_t nchunks = p.chunk_off1[g.N];
@@ -914,7 +913,7 @@ __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const floa
             // pairs of tiles per wave (fetch_pair)
             auto tile = [&](int32_t i, const float (&x4)[4], float gy) {
                 const bool valid = i < wn;
-                const f32x16 dx = tile_backward_mfma<P, H, NEAT_ACT_SILU>(w, x4, gy, valid, NEAT_ACT_SOFTPLUS, g.beta, sb, acc);
+                const f32x16 dx = tile_backward_mfma<H, NEAT_ACT_SILU>(w, x4, gy, valid, NEAT_ACT_SOFTPLUS, g.beta, sb, acc);
                 if (valid)
                 {
                     // [2][S][4]: channel halves
@@ -926,7 +925,7 @@ __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const floa
             for (int32_t p0 = wave * 64; p0 < wn; p0 += 256)
             {
                 PairIn cur;
-                fetch_pair<P::kBF16, true>(g, cx, p0, w0, wn, base, nb, ngrid, sgc, cur);
+                fetch_pair<false, true>(g, cx, p0, w0, wn, base, nb, ngrid, sgc, cur);
                 // one copy of the tile code for both halves of the pair (smaller code, fewer live registers)
 #pragma unroll 1
                 for (int h = 0; h < 2; ++h)

@@ -36,10 +36,10 @@ __device__ __forceinline__ void transpose_frags(unsigned short* tile, const bf16
     sf[1] = tr_load(tile, 1);
 }
 
-// Backward of one tile of 32 samples: the values of tile_backward_mfma<PrecBF16, H, NEAT_ACT_SILU> step by step (the same
-// roundings to BF16, the same products in the same order up to dL/dx), with each activation and its derivative taken
-// once, right behind the pre-activation, and the operands of the weight gradients (which contract over the samples)
-// taken from LDS transposes of the fragments the other products use. Returns dL/dx in registers 0..3. stash: this wave's 64 H / 8 float4 in LDS.
+// Backward of one tile of 32 samples: the steps of tile_backward_mfma in BF16 (every operand of a product rounded once,
+// the products in the same order up to dL/dx), with each activation and its derivative taken once, right behind the
+// pre-activation, and the operands of the weight gradients (which contract over the samples) taken from LDS transposes
+// of the fragments the other products use. Returns dL/dx in registers 0..3. stash: this wave's 64 H / 8 float4 in LDS.
 template <int H>
 __device__ __forceinline__ f32x16 tile_backward_bf16(const WeightLDS<PrecBF16, H>& w, const float (&x4)[4], float gy,
                                                      bool valid, float beta, unsigned short* tile, float4* stash,

@@ -274,9 +274,9 @@ __global__ void __launch_bounds__(256) k_prop_bwd(PropSegs sg, const float* __re
 #pragma unroll
         for (int st = 0; st < 2; ++st)
         {
-            const auto a = stage_frag<PrecBF16>(sA, n, st, g, false);
-            dW1          = PrecBF16::mma(a, stage_frag<PrecBF16>(sB, n, st, g, false), dW1);
-            E            = PrecBF16::mma(a, stage_frag<PrecBF16>(sX, n, st, g, n != 7), E);
+            const auto a = stage_frag(sA, n, st, g, false);
+            dW1          = PrecBF16::mma(a, stage_frag(sB, n, st, g, false), dW1);
+            E            = PrecBF16::mma(a, stage_frag(sX, n, st, g, n != 7), E);
         }
         wave_lds_fence();
         // phase 2: E(cols 0..6) += dZ1 [x; 1]^T
@@ -285,7 +285,7 @@ __global__ void __launch_bounds__(256) k_prop_bwd(PropSegs sg, const float* __re
         wave_lds_fence();
 #pragma unroll
         for (int st = 0; st < 2; ++st)
-            E = PrecBF16::mma(stage_frag<PrecBF16>(sA, n, st, g, false), stage_frag<PrecBF16>(sX, n, st, g, n > 6), E);
+            E = PrecBF16::mma(stage_frag(sA, n, st, g, false), stage_frag(sX, n, st, g, n > 6), E);
         wave_lds_fence();
         // phase 3: dW2 += dl relu(z2)^T (rows 0..7)
 #pragma unroll
@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(256) k_prop_bwd(PropSegs sg, const float* __re
         wave_lds_fence();
 #pragma unroll
         for (int st = 0; st < 2; ++st)
-            dW2 = PrecBF16::mma(stage_frag<PrecBF16>(sA, n, st, g, n >= kPOut), stage_frag<PrecBF16>(sB, n, st, g, false),
+            dW2 = PrecBF16::mma(stage_frag(sA, n, st, g, n >= kPOut), stage_frag(sB, n, st, g, false),
                                 dW2);
         wave_lds_fence();
     }
