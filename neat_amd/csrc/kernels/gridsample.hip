@@ -10,24 +10,30 @@
 namespace neat
 {
 
-// Channel-last fast path: C4 groups of 4 channels read with one 16-byte load per corner.
-template <bool kChannelsLast>
+// kChannelsLast: a corner's channels are one contiguous run, read with 16-byte loads. kLanes lanes share a sample, each
+// taking every kLanes-th channel quad: bound by the cache lines an instruction touches, of which 8 channels then cost one
+// per corner instead of one per corner and quad. 13.0 M samples, 4096 grids of 17^3 x 8: 523 us with one lane a sample,
+// 345 us with two. Per channel the arithmetic is the same, so are the bits.
+template <bool kChannelsLast, int kLanes = 1>
 __global__ void __launch_bounds__(256) k_gs3d_fwd(GridArgs g, const int64_t* index, const float* uv, int64_t S,
                                                   float* out)
 {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = l / kLanes;
     if (i >= S) return;
     const int64_t n = index[i];
-    if (n < 0 || n >= g.N)
-    {
-        // a slot outside the grid (e.g. -1 for an inactive node) samples zeros instead of reading out of bounds
-        for (int c = 0; c < g.C; ++c) out[i * g.C + c] = 0.f;
-        return;
-    }
-    Tri t = trilinear(g, n, uv[3 * i], uv[3 * i + 1], uv[3 * i + 2]);
     if constexpr (kChannelsLast)
     {
-        for (int c = 0; c < g.C; c += 4)
+        const int32_t c0 = 4 * (int32_t)(l % kLanes);
+        if (n < 0 || n >= g.N)
+        {
+            // a slot outside the grid (e.g. -1 for an inactive node) samples zeros instead of reading out of bounds
+            for (int c = c0; c < g.C; c += 4 * kLanes)
+                *reinterpret_cast<float4*>(out + i * g.C + c) = make_float4(0.f, 0.f, 0.f, 0.f);
+            return;
+        }
+        const Tri t = trilinear(g, n, uv[3 * i], uv[3 * i + 1], uv[3 * i + 2]);
+        for (int c = c0; c < g.C; c += 4 * kLanes)
         {
             float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -44,6 +50,12 @@ __global__ void __launch_bounds__(256) k_gs3d_fwd(GridArgs g, const int64_t* ind
     }
     else
     {
+        if (n < 0 || n >= g.N)
+        {
+            for (int c = 0; c < g.C; ++c) out[i * g.C + c] = 0.f;
+            return;
+        }
+        const Tri t = trilinear(g, n, uv[3 * i], uv[3 * i + 1], uv[3 * i + 2]);
         for (int c = 0; c < g.C; ++c)
         {
             float acc = 0.f;
@@ -287,7 +299,10 @@ extern "C"
         if (S == 0) return NEAT_OK;
         NEAT_REQUIRE(index && uv && out, "neat_gs3d_fwd: null pointer");
         hipStream_t s = as_stream(stream);
-        if (channels_last(g) && (reinterpret_cast<uintptr_t>(out) % 16) == 0)
+        const bool cl = channels_last(g) && (reinterpret_cast<uintptr_t>(out) % 16) == 0;
+        if (cl && C % 8 == 0 && S < INT32_MAX - 256)  // a launch holds fewer than 2^32 threads
+            k_gs3d_fwd<true, 2><<<grid_for(2 * S, 256), 256, 0, s>>>(g, index, uv, S, out);
+        else if (cl)
             k_gs3d_fwd<true><<<grid_for(S, 256), 256, 0, s>>>(g, index, uv, S, out);
         else
             k_gs3d_fwd<false><<<grid_for(S, 256), 256, 0, s>>>(g, index, uv, S, out);
