@@ -79,8 +79,11 @@ struct WeightLDSSplitFwd
     uint32_t norm[4];
 };
 
-// Packed parameter layout as load_weights (C = 8). Ends in a barrier.
-template <int H>
+// Packed parameter layout as load_weights (C = 8). Ends in a barrier. kRelu (relu decoders only): a unit without any
+// weight or bias gets the bias -1, which leaves it as inactive as its pre-activation of exactly zero would; at zero it
+// would send every tile of the backward to the plain evaluation. On the trained bench field, most of whose units are
+// such: FP32 step of 53.7 M samples 19.0 ms with the zeros, 13.7 ms like this.
+template <int H, bool kRelu = false>
 __device__ void load_weights_split_fwd(const float* params, WeightLDSSplitFwd<H>& w)
 {
     constexpr int MT = H / 32, C = 8;
@@ -112,6 +115,8 @@ __device__ void load_weights_split_fwd(const float* params, WeightLDSSplitFwd<H>
             atomicMax(&w.norm[1], __float_as_uint(fabsf(b0[r])));
             atomicMax(&w.norm[2], __float_as_uint(a1));
             atomicMax(&w.norm[3], __float_as_uint(fabsf(b1[r])));
+            w.vec[0][r] = kRelu && a0 == 0.f && b0[r] == 0.f ? -1.f : b0[r];
+            w.vec[1][r] = kRelu && a1 == 0.f && b1[r] == 0.f ? -1.f : b1[r];
         }
     }
     for (int t = threadIdx.x; t < MT * 64; t += blockDim.x)
@@ -143,8 +148,7 @@ __device__ void load_weights_split_fwd(const float* params, WeightLDSSplitFwd<H>
     }
     for (int t = threadIdx.x; t < 64; t += blockDim.x)
     {
-        w.vec[0][t] = t < H ? b0[t] : 0.f;
-        w.vec[1][t] = t < H ? b1[t] : 0.f;
+        if (t >= H) w.vec[0][t] = w.vec[1][t] = 0.f;
         w.vec[2][t] = t < H ? W2[t] : 0.f;
         w.vec[3][t] = t == 0 ? b2[0] : 0.f;
     }
@@ -345,7 +349,7 @@ __device__ void load_weights_split(const float* __restrict__ params, float* copy
     const float* W0 = copy;
     const float* W1 = W0 + H * C + H;
     const float* W2 = W1 + H * H + H;
-    load_weights_split_fwd<H>(copy, w);
+    load_weights_split_fwd<H, true>(copy, w);
     for (int t = threadIdx.x; t < MT * MT * 2 * 64; t += blockDim.x)
     {
         const int l = t % 64, st = (t / 64) % 2, ms = (t / 128) % MT, mt = t / (128 * MT);
