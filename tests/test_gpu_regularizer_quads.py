@@ -56,3 +56,6 @@ def test_edge_two_quads(C):
     assert abs(la.item() - lb.item()) <= 1e-6 * abs(lb.item())
     # a few roundings of 2^-24 per term, in another order
     assert float((ga.double() - gb.double()).norm() / gb.double().norm()) <= 1e-6
+    # the loss alone sums in the same order
+    lo = ops.edge_loss_direct(*d, flags, pre, tid, grid, 9, 1e-3)
+    assert lo.item() == la.item()
