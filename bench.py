@@ -291,17 +291,16 @@ def main():
     fwd_flop = 2 * (C * H + H * H + H * 1)  # decoder forward per sample, 2 FLOP per MAC
     mm_peak = BF16_PEAK_TFLOPS if (a.path == "fused" and a.precision == "bf16") else FP32_PEAK_TFLOPS
     mm = "fp32_valu" != a.precision
-    prec_tag = {"bf16": "PrecBF16", "fp32": "PrecF32"}.get(a.precision)
     act = 1 if cfg.act == "relu" else 2
     grid_bytes = ds.grid.numel() * 4
-    if not (mm and prec_tag):
-        bwd_kernel = f"k_proj_bw1<{C},{H}>"
-    elif prec_tag == "PrecBF16" and cfg.act == "relu":
-        bwd_kernel = f"k_mfma_bwd_relu<{H}>"
+    if not mm:
+        fwd_kernel, bwd_kernel = f"k_proj_fwd<{C},{H},{act}>", f"k_proj_bw1<{C},{H}>"
+    elif a.precision == "bf16":
+        form = "k_mfma_%s_relu" if cfg.act == "relu" else "k_bf16_%s"
+        fwd_kernel, bwd_kernel = f"{form % 'fwd'}<{H}>", f"{form % 'bwd'}<{H}>"
     else:
-        bwd_kernel = f"k_mfma_bwd<{prec_tag},{H},{act}>"
-    fwd_kernel = (f"k_mfma_fwd_relu<{H}>" if prec_tag == "PrecBF16" and cfg.act == "relu" else
-                  f"k_mfma_fwd<{prec_tag},{H},{act}>" if mm and prec_tag else f"k_proj_fwd<{C},{H},{act}>")
+        fwd_kernel = f"k_split_fwd<{H},{act}>"
+        bwd_kernel = f"k_split_bwd<{H}>" if cfg.act == "relu" else f"k_mfma_bwd<{H}>"
     # algorithmic work per launch of each stage's dominant kernel (per-unit figure x the units of one launch):
     # decoder FLOPs per sample (backward: 2x the forward, no recomputation counted); the scatter reads 16 B of
     # dL/dfeature per sample and writes the gradient grid once
