@@ -140,9 +140,9 @@ __global__ void __launch_bounds__(kDecBwdThreads, 2) k_dec_split_bwd(const float
     write_split_partials<H>(params, w, acc, stage, partials + (int64_t)blockIdx.x * P_total);
 }
 
-// Backward for silu on the FP32 matrix cores; one partial slice per wave (kDecMfmaWaves per workgroup).
+// Backward for silu on the FP32 matrix cores; one partial slice per wave (at most kDecMfmaWaves per workgroup).
 template <int H, int ACT>
-__global__ void __launch_bounds__(256) k_dec_mfma_bwd(const float* __restrict__ x, int64_t S,
+__global__ void __launch_bounds__(64 * kDecMfmaWaves) k_dec_mfma_bwd(const float* __restrict__ x, int64_t S,
                                                       const float* __restrict__ params, int last_act, float beta,
                                                       const float* __restrict__ gy, float* __restrict__ gx,
                                                       float* __restrict__ partials, int32_t P_total)
@@ -151,12 +151,12 @@ __global__ void __launch_bounds__(256) k_dec_mfma_bwd(const float* __restrict__ 
     __shared__ WeightLDS<P, H> w;
     __shared__ __align__(16) float stage[kDecMfmaWaves][Stage::elems(H)];
     load_weights<P, H, 8>(params, w);
-    const int l = threadIdx.x & 63, wave = threadIdx.x >> 6, hg = l >> 5;
+    const int l = threadIdx.x & 63, wave = threadIdx.x >> 6, hg = l >> 5, waves = blockDim.x >> 6;
     BwdStage<H> sb(stage[wave]);
     BwdAcc<H / 32> acc;
     __syncthreads();
     const int64_t tiles = (S + 31) / 32;
-    for (int64_t t = (int64_t)blockIdx.x * kDecMfmaWaves + wave; t < tiles; t += (int64_t)gridDim.x * kDecMfmaWaves)
+    for (int64_t t = (int64_t)blockIdx.x * waves + wave; t < tiles; t += (int64_t)gridDim.x * waves)
     {
         const int64_t i  = t * 32 + (l & 31);
         const bool valid = i < S;
@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(256) k_dec_mfma_bwd(const float* __restrict__ 
             for (int j = 0; j < 4; ++j) gx[i * 8 + 4 * hg + j] = dx[j];
         }
     }
-    write_param_partials<H, 8>(acc, partials + ((int64_t)blockIdx.x * kDecMfmaWaves + wave) * P_total);
+    write_param_partials<H, 8>(acc, partials + ((int64_t)blockIdx.x * waves + wave) * P_total);
 }
 
 // the shapes the matrix-core form covers
@@ -287,21 +287,25 @@ extern "C"
         float* partials = wt + P;
         if (dec_mfma(in, hidden, layers, out, act))
         {
-            // one slice per workgroup (relu) or kDecMfmaWaves, within the bwd_workgroups(S) slices the workspace holds
+            // one slice per workgroup (relu) or per wave (silu), within the bwd_workgroups(S) slices the workspace
+            // holds: with fewer than kDecMfmaWaves of those the one workgroup has as many waves as there are slices
             int wg = std::min(bwd_workgroups(S), device_cus()), slices = wg;
+            const int waves = std::min(bwd_workgroups(S), kDecMfmaWaves);
             if (act != NEAT_ACT_RELU)
             {
                 wg     = std::max(1, std::min(bwd_workgroups(S) / kDecMfmaWaves, device_cus()));
-                slices = wg * kDecMfmaWaves;
+                slices = wg * waves;
             }
             if (hidden == 32 && act == NEAT_ACT_RELU)
                 k_dec_split_bwd<32><<<wg, kDecBwdThreads, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
             else if (act == NEAT_ACT_RELU)
                 k_dec_split_bwd<64><<<wg, kDecBwdThreads, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
             else if (hidden == 32)
-                k_dec_mfma_bwd<32, NEAT_ACT_SILU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
+                k_dec_mfma_bwd<32, NEAT_ACT_SILU><<<wg, 64 * waves, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials,
+                                                                           P);
             else
-                k_dec_mfma_bwd<64, NEAT_ACT_SILU><<<wg, 256, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
+                k_dec_mfma_bwd<64, NEAT_ACT_SILU><<<wg, 64 * waves, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials,
+                                                                           P);
             NEAT_LAUNCHED();
             k_dec_reduce_partials<<<reduce_partials_blocks(P), 256, 0, s>>>(partials, slices, P, gparams);
             NEAT_LAUNCHED();
