@@ -393,7 +393,8 @@ struct SplitStage
     unsigned short plane[3][32 * kTrRow];
 };
 
-// A wave's running parameter-gradient products: G = [Z2 > 0] (dz h1)^T (the hidden-weight gradient without its row
+// A wave's running parameter-gradient products, of every other wave with the opposite sign (so that the accumulation's
+// rounding down cancels between them): G = [Z2 > 0] (dz h1)^T (the hidden-weight gradient without its row
 // factor w3), E (columns as T), and the output bias's. The output-weight gradient follows from them at the end:
 // sum_n h2[r] dz = sum_n [z2[r] > 0] z2[r] dz = sum_c W1[r][c] G[r][c] + b1[r] (sum_n [z2[r] > 0] dz).
 template <int MT>
@@ -401,8 +402,8 @@ struct SplitAcc
 {
     f32x16 G[MT][MT];
     f32x16 E[MT];
-    float b3;
-    __device__ SplitAcc() : b3(0.f)
+    float b3, sign;
+    __device__ SplitAcc() : b3(0.f), sign((blockIdx.x + (threadIdx.x >> 6)) & 1 ? -1.f : 1.f)
     {
 #pragma unroll
         for (int a = 0; a < MT; ++a)
@@ -508,7 +509,7 @@ __device__ __forceinline__ void tile_backward_split(const float* __restrict__ pa
         for (int i = 0; i < 16; ++i) z = fmaf(w3[i], act_f(NEAT_ACT_RELU, z2[mt][i], beta), z);
     }
     z = z + __shfl_xor(z, 32) + w.vec[3][0];
-    const float dz = valid ? gy * act_d(last_act, z, beta) : 0.f;
+    const float dz = valid ? acc.sign * (gy * act_d(last_act, z, beta)) : 0.f;
     if (hg == 0) acc.b3 += dz;
     // T
     unsigned short* T = sg.plane[0];
@@ -582,7 +583,7 @@ __device__ __forceinline__ void tile_backward_split(const float* __restrict__ pa
     }
     // the three row groups of W0's planes
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dx[j] = xa[j] + (xa[j + 4] + xa[j + 8]);
+    for (int j = 0; j < 4; ++j) dx[j] = acc.sign * (xa[j] + (xa[j + 4] + xa[j + 8]));
     // the hidden layer's gradients
     bf16x8 ms_[MT][2][1];
 #pragma unroll
@@ -621,13 +622,16 @@ constexpr int split_sums()
     return H * H + 32 * H + 1;
 }
 
-// A wave's sums written to `red` (add: added to it).
+// A wave's sums, with their sign put right, written to `red` (add: added to it).
 template <int H>
 __device__ __forceinline__ void put_split_sums(SplitAcc<H / 32>& acc, float* red, bool add)
 {
     constexpr int MT = H / 32;
     const int l = threadIdx.x & 63, n = l & 31, hg = l >> 5;
-    auto put = [&](int i, float v) { red[i] = add ? red[i] + v : v; };
+    auto put = [&](int i, float v) {
+        v *= acc.sign;
+        red[i] = add ? red[i] + v : v;
+    };
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
     {
