@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(kDecBwdThreads, 2) k_dec_split_bwd(const float
             for (int j = 0; j < 4; ++j) gx[i * 8 + 4 * hg + j] = dx[j];
         }
     }
-    write_split_partials<H>(params, w, acc, stage, partials + (int64_t)blockIdx.x * P_total);
+    write_split_partials<H>(w, acc, stage, partials + (int64_t)blockIdx.x * P_total);
 }
 
 // Backward for silu on the FP32 matrix cores; one partial slice per wave (at most kDecMfmaWaves per workgroup).

@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(kSplitThreads, 2) k_split_bwd(ProjGeom g, Plan
             __syncthreads();
         }
     }
-    write_split_partials<H>(params, w, acc, stage, partials + (int64_t)blockIdx.x * P_total);
+    write_split_partials<H>(w, acc, stage, partials + (int64_t)blockIdx.x * P_total);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
     if (l == 0) atomicMax(dmax, __float_as_uint(amax));  // non-negative floats order like their bit patterns

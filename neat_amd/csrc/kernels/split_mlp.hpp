@@ -399,15 +399,21 @@ struct SplitStage
 
 // A wave's running parameter-gradient products, of every other wave with the opposite sign (so that the accumulation's
 // rounding down cancels between them): G = [Z2 > 0] (dz h1)^T (the hidden-weight gradient without its row
-// factor w3), E (columns as T), and the output bias's. The output-weight gradient follows from them at the end:
-// sum_n h2[r] dz = sum_n [z2[r] > 0] z2[r] dz = sum_c W1[r][c] G[r][c] + b1[r] (sum_n [z2[r] > 0] dz).
+// factor w3), E (columns as T), and the output layer's: the bias's on every lane of the lower half, the weights' h2 dz
+// summed over the tile, one row per lane (transpose_sum).
+//
+// The output weights' gradient also follows from G, as sum_c W1[r][c] G[r][c] + b1[r] (sum_n [z2[r] > 0] dz), but keeps
+// G's roundings at the size of its terms: with biases that cancel the sums over c to a tenth / a hundredth and output
+// gradients of one sign (H = 64, 10^6 rows) 1.4e-7 / 8.0e-7 from 64 bits, where the FP32 matrix cores gave 0.7e-7 /
+// 0.8e-7 and these sums give 0.6e-7 / 1.2e-7. They take 11 of 191 us there, and 0.45 of 15.0 ms of the projector's FP32
+// step of 53.3 M samples.
 template <int MT>
 struct SplitAcc
 {
     f32x16 G[MT][MT];
     f32x16 E[MT];
-    float b3, sign;
-    __device__ SplitAcc() : b3(0.f), sign((blockIdx.x + (threadIdx.x >> 6)) & 1 ? -1.f : 1.f)
+    float b3, w3, sign;
+    __device__ SplitAcc() : b3(0.f), w3(0.f), sign((blockIdx.x + (threadIdx.x >> 6)) & 1 ? -1.f : 1.f)
     {
 #pragma unroll
         for (int a = 0; a < MT; ++a)
@@ -442,6 +448,50 @@ __device__ __forceinline__ float min_abs(const f32x16& a)
 #pragma unroll
     for (int i = 1; i < 16; ++i) m = fminf(m, fabsf(a[i]));
     return m;
+}
+
+// x of lane l ^ B of the same 16-lane row (B = 4: of lane l ^ 7)
+template <int B>
+__device__ __forceinline__ float lane_xor(float x)
+{
+    constexpr int kCtl = B == 1 ? 0xB1 : (B == 2 ? 0x4E : (B == 4 ? 0x141 : 0x128));  // quad_perm, half mirror, ror:8
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), kCtl, 0xF, 0xF, true));
+}
+
+// One step of transpose_sum: the lane keeps the lower or the upper half of the first 2 N values, by bit B of its number, and
+// adds its partner's.
+template <int B, int N>
+__device__ __forceinline__ void transpose_step(float* v)
+{
+    const bool up = threadIdx.x & B;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+    {
+        const float keep = up ? v[i + N] : v[i], give = up ? v[i] : v[i + N];
+        v[i]             = keep + lane_xor<B>(give);
+    }
+}
+
+// The sum of value j = n / (32 / N) over the 32 lanes of each half wave, on lane n of the half, of N = 16 or 32 values per
+// lane: halving the values in every step takes about 3 N instructions, the N sums one by one 5 N.
+template <int N>
+__device__ __forceinline__ float transpose_sum(float (&v)[N])
+{
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i)
+    {
+        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + N / 2]), false,
+                                                        false);
+        v[i] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    }
+    transpose_step<8, N / 4>(v);
+    transpose_step<4, N / 8>(v);
+    transpose_step<2, N / 16>(v);
+    if constexpr (N == 32)
+        transpose_step<1, 1>(v);
+    else
+        v[0] += lane_xor<1>(v[0]);
+    return v[0];
 }
 
 // Backward of one tile of 32 samples on a wave (arguments as tile_backward_mfma): adds the tile's parameter-gradient
@@ -532,6 +582,14 @@ __device__ __forceinline__ void tile_backward_split(const float* __restrict__ pa
     z = z + __shfl_xor(z, 32) + w.vec[3][0];
     const float dz = valid ? acc.sign * (gy * act_d(last_act, z, beta)) : 0.f;
     if (hg == 0) acc.b3 += dz;
+    {
+        float v[16 * MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v[16 * mt + i] = act_f(NEAT_ACT_RELU, z2[mt][i], beta) * dz;
+        acc.w3 += transpose_sum(v);
+    }
     // T
     unsigned short* T = sg.plane[0];
     {
@@ -636,11 +694,11 @@ __device__ __forceinline__ void tile_backward_split(const float* __restrict__ pa
     }
 }
 
-// Floats of a wave's sums as put_split_sums lays them out: G [H][H], E [H][32], b3.
+// Floats of a wave's sums as put_split_sums lays them out: G [H][H], E [H][32], w3 [H], b3.
 template <int H>
 constexpr int split_sums()
 {
-    return H * H + 32 * H + 1;
+    return H * H + 33 * H + 1;
 }
 
 // A wave's sums, with their sign put right, written to `red` (add: added to it).
@@ -668,15 +726,17 @@ __device__ __forceinline__ void put_split_sums(SplitAcc<H / 32>& acc, float* red
     float b3 = acc.b3;
 #pragma unroll
     for (int off = 16; off >= 1; off >>= 1) b3 += __shfl_xor(b3, off);
-    if (l == 0) put(H * H + 32 * H, b3);
+    if (l == 0) put(H * H + 33 * H, b3);
+    const int j = n / (2 / MT);  // transpose_sum's value on this lane
+    if (n % (2 / MT) == 0) put(H * H + 32 * H + 32 * (j / 16) + crow(j % 16, hg), acc.w3);
 }
 
 // The workgroup's parameter-gradient slice, in the packed layout: its waves' sums added in a fixed order in LDS (in the
 // transpose tiles, which are done with; as many waves at a time as have room there), the hidden layer's rows times
-// w3, the output weights' gradient from them (SplitAcc), then stored. NW waves; called by every thread.
+// w3, then stored. NW waves; called by every thread.
 template <int H, int NW>
-__device__ __forceinline__ void write_split_partials(const float* __restrict__ params, const WeightLDSSplit<H>& w,
-                                                     SplitAcc<H / 32>& acc, SplitStage (&stage)[NW], float* part)
+__device__ __forceinline__ void write_split_partials(const WeightLDSSplit<H>& w, SplitAcc<H / 32>& acc,
+                                                     SplitStage (&stage)[NW], float* part)
 {
     constexpr int C = 8, ob0 = H * C, oW1 = ob0 + H, ob1 = oW1 + H * H, oW2 = ob1 + H, ob2 = oW2 + H;
     constexpr int Q = split_sums<H>(), kFit = (int)(sizeof(stage) / (Q * sizeof(float))), NS = kFit < NW ? kFit : NW;
@@ -704,25 +764,14 @@ __device__ __forceinline__ void write_split_partials(const float* __restrict__ p
         part[t]        = e[0] + (e[8] + e[16]);
     }
     for (int t = threadIdx.x; t < H * H; t += blockDim.x) part[oW1 + t] = red[t] * w.vec[2][t / H];
-    // 8 lanes to a row
-    for (int t = threadIdx.x; t < 8 * H; t += blockDim.x)
+    for (int r = threadIdx.x; r < H; r += blockDim.x)
     {
-        const int r    = t >> 3, q = t & 7;
         const float* e = E + r * 32 + kTDz;
-        const float gb = e[0] + (e[1] + e[2]);
-        float v        = q == 0 ? w.vec[1][r] * gb : 0.f;
-#pragma unroll
-        for (int c = 0; c < H; c += 8) v = fmaf(params[oW1 + r * H + c + q], red[r * H + c + q], v);
-#pragma unroll
-        for (int off = 4; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-        if (q == 0)
-        {
-            part[ob0 + r] = E[r * 32 + kTOnes];
-            part[ob1 + r] = gb * w.vec[2][r];
-            part[oW2 + r] = v;
-        }
+        part[ob0 + r]  = E[r * 32 + kTOnes];
+        part[ob1 + r]  = (e[0] + (e[1] + e[2])) * w.vec[2][r];
+        part[oW2 + r]  = E[32 * H + r];
     }
-    if (threadIdx.x == 0) part[ob2] = E[32 * H];
+    if (threadIdx.x == 0) part[ob2] = E[33 * H];
 }
 
 }  // namespace neat

@@ -15,12 +15,12 @@ DEV = "cuda"
 S = 50021
 
 
-def cancelling(H, seed):
+def cancelling(H, seed, scale=0.3):
     g = torch.Generator(device=DEV).manual_seed(seed)
     rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
     W0, b0, W1 = rnd(H, 8) / 8 ** 0.5, 0.3 * rnd(H).abs() + 0.5, (rnd(H, H) * (2 / H) ** 0.5).abs()
     W2, b2 = rnd(1, H) * (2 / H) ** 0.5, 0.3 * rnd(1)
-    x = 0.3 * rnd(S, 8)
+    x = scale * rnd(S, 8)
     b1 = -(torch.relu(x @ W0.T + b0) @ W1.T).mean(0)
     return x, (W0, b0, W1, b1, W2, b2)
 
@@ -46,3 +46,26 @@ def test_forward(seed, H):
     packed = torch.cat([t.reshape(-1) for t in p])
     got = ops.decoder_fwd(x, packed, 8, H, 1, 1, "relu", "id", 2.0)
     assert float((got.double() - want).norm()) <= float((plain.double() - want).norm())
+
+
+@pytest.mark.parametrize("H", [32, 64])
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_output_weight_gradient(seed, H):
+    """sum_n h2 dy of output gradients of one sign, against the same sum of the plain evaluation's h2, each product and
+    addition rounded (pairwise sums of 2^16 terms: 16 roundings more, 2^-24 of the sum each, sqrt(16) of them allowed for).
+    Rows with a unit within rounding of zero are left out: a unit is rounded like its pre-activation there."""
+    print("case: cancelling decoder, output weights", seed, H, flush=True)
+    x, p = cancelling(H, seed, scale=0.05)
+    W0, b0, W1, b1, W2, b2 = (t.double() for t in p)
+    z1 = x.double() @ W0.T + b0
+    z2 = torch.relu(z1) @ W1.T + b1
+    clear = (z1.abs() > 1e-5).all(1) & (z2.abs() > 1e-4).all(1)
+    gy = torch.rand(S, 1, device=DEV, generator=torch.Generator(device=DEV).manual_seed(9)) * clear[:, None]
+    want = (torch.relu(z2) * gy.double()).sum(0)
+    h2 = torch.relu(fp32_layer(torch.relu(fp32_layer(x, p[0], p[1])), p[2], p[3]))
+    plain = (h2 * gy).double().sum(0)
+    packed = torch.cat([t.reshape(-1) for t in p])
+    gp, _ = ops.decoder_bwd(x, packed, gy, 8, H, 1, 1, "relu", "id", 2.0)
+    got = gp[-1 - H:-1].double()
+    bar = float((plain - want).norm()) + 4 * 2.0 ** -24 * float(want.norm())
+    assert float((got - want).norm()) <= bar
