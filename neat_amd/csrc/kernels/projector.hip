@@ -559,6 +559,23 @@ __global__ void __launch_bounds__(kScatterThreads) k_proj_bw2(ProjGeom g, Plan p
 #pragma unroll
             for (int k = 0; k < 8; ++k) acc[k][0] = acc[k][1] = acc[k][2] = acc[k][3] = 0.f;
             auto flush = [&]() {
+                if constexpr (decltype(fast)::value)
+                {
+                    // a gradient or coordinate that is not finite leaves its channel's eight sums not finite: they add
+                    // nothing, as a NaN does in the general conversion (a bit pattern less the constant's would be a
+                    // huge finite value)
+                    const auto finite = [&](int q) { return fabsf(acc[0][q]) < INFINITY; };
+                    if (!(finite(0) && finite(1) && finite(2) && finite(3)))
+                    {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            if (!finite(q))
+                            {
+#pragma unroll
+                                for (int k = 0; k < 8; ++k) acc[k][q] = 0.f;
+                            }
+                    }
+                }
                 const int vz[2] = {cz0 * G * G, cz1 * G * G}, vy[2] = {cy0 * G, cy1 * G}, vx[2] = {cx0, cx1};
 #pragma unroll
                 for (int k = 0; k < 8; ++k)
@@ -631,8 +648,9 @@ __global__ void __launch_bounds__(kScatterThreads) k_proj_bw2(ProjGeom g, Plan p
             if (cell >= 0) flush();
         };
         // a run of at most 64 samples stays within to_fixed's range: chunks of more than 64 samples per lane (a
-        // segment longer than a chunk) and non-finite gradients take the general conversion
-        if (L2 <= 64 && isfinite(__uint_as_float(*dmax)))
+        // segment longer than a chunk) take the general conversion, and batches with an infinite gradient or one whose
+        // sums could overflow. (A NaN does not show in the largest gradient: flush looks for it.)
+        if (L2 <= 64 && __uint_as_float(*dmax) < 0x1p100f)
             walk(std::true_type{});
         else
             walk(std::false_type{});
