@@ -280,12 +280,10 @@ struct RayScratch
     int64_t ray_stride, seg_stride;
 };
 
-__global__ void __launch_bounds__(128) k_ray_walk(TreeArgs T, const float* ro, const float* rd, int64_t R,
-                                                  int32_t max_spn, RayScratch sc, int64_t* nseg, int64_t* nsamp,
-                                                  int32_t* max_per_ray)
+// One thread's ray: its segments into the scratch, its counts.
+__device__ __forceinline__ void walk_ray(const TreeArgs& T, const float* ro, const float* rd, int64_t r, int32_t max_spn,
+                                         const RayScratch& sc, int64_t* nseg, int64_t* nsamp, int32_t* max_per_ray)
 {
-    int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= R) return;
     float o[3], d[3];
     load_ray(ro, rd, r, o, d);
     int64_t nk, ns;
@@ -296,12 +294,24 @@ __global__ void __launch_bounds__(128) k_ray_walk(TreeArgs T, const float* ro, c
     if (max_per_ray) atomicMax(max_per_ray, (int32_t)ns);
 }
 
+__global__ void __launch_bounds__(128) k_ray_walk(TreeArgs T, const float* ro, const float* rd, int64_t R,
+                                                  int32_t max_spn, RayScratch sc, int64_t* nseg, int64_t* nsamp,
+                                                  int32_t* max_per_ray)
+{
+    int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < R) walk_ray(T, ro, rd, r, max_spn, sc, nseg, nsamp, max_per_ray);
+}
+
 // One wave per ray, for batches too small to fill the chip with one thread per ray: the octree level by level, the lanes
 // testing the children of the level's hit nodes that have active descendants. A child is tested exactly when the
 // stackless walk would visit it (its parent is hit and has an active descendant), with the same box (halved from the
 // parent's) and the same slab test, so the segments are the same; they are put in canonical order by ranking each
 // against the others. A ray with more than kCoopSegs segments, or more than kCoopNodes nodes to expand on one level
 // (rays along faces touch both sides of them), is walked by one lane instead.
+//
+// The boxes are the same where halving and doubling them is exact (exact_boxes), as in a tree of [-1, 1]^3. In any other
+// the thread walk's depend on the way it took, and the rays are walked by a thread each, as in larger batches and in
+// the other passes over the tree.
 //
 // The walk is a chain of dependent steps, about 300 per ray in a depth-5 tree, whose latency a small batch does not
 // hide; here it is one round per 64 children. A thread per ray costs less work in all, hence the limit in coop_rays
@@ -310,6 +320,24 @@ constexpr int kCoopWaves = 4;
 constexpr int kCoopNodes = 128;
 constexpr int kCoopSegs  = 128;
 
+// Whether every box down to `depth` comes out of halving exactly, and its parent's out of doubling it: with the root's
+// corners below 2^e and multiples of 2^u, the corners are multiples of 2^(u - depth), and so are the sums of two, which
+// are below 2^(e + 1): 24 bits hold them for u >= e + depth - 23.
+__device__ __forceinline__ bool exact_boxes(const TreeArgs& T, int32_t depth)
+{
+    bool exact = true;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+    {
+        const float a = T.pmin[k], b = T.pmax[k], m = fmaxf(fabsf(a), fabsf(b));
+        int e;
+        frexpf(m, &e);
+        const float x = ldexpf(a, 23 - e - depth), y = ldexpf(b, 23 - e - depth);
+        exact = exact && m > 1e-30f && m < 1e30f && x == rintf(x) && y == rintf(y);
+    }
+    return exact;
+}
+
 struct CoopList
 {
     int32_t node[kCoopNodes];
@@ -317,9 +345,16 @@ struct CoopList
 };
 
 __global__ void __launch_bounds__(64 * kCoopWaves) k_ray_coop(TreeArgs T, const float* ro, const float* rd, int64_t R,
-                                                              int32_t max_spn, RayScratch sc, int64_t* nseg,
-                                                              int64_t* nsamp, int32_t* max_per_ray)
+                                                              int32_t max_spn, int32_t max_depth, RayScratch sc,
+                                                              int64_t* nseg, int64_t* nsamp, int32_t* max_per_ray)
 {
+    if (!exact_boxes(T, max_depth))
+    {
+        // the grid has 64 times the threads this takes
+        const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+        if (r < R) walk_ray(T, ro, rd, r, max_spn, sc, nseg, nsamp, max_per_ray);
+        return;
+    }
     __shared__ CoopList s_list[kCoopWaves][2];
     __shared__ int32_t s_node[kCoopWaves][kCoopSegs], s_cnt[kCoopWaves][kCoopSegs];
     __shared__ float s_tmin[kCoopWaves][kCoopSegs], s_tmax[kCoopWaves][kCoopSegs];
@@ -404,15 +439,7 @@ __global__ void __launch_bounds__(64 * kCoopWaves) k_ray_coop(TreeArgs T, const 
     over = over || k > kCoopSegs;
     if (over)
     {
-        if (l == 0)
-        {
-            int64_t nk, nn;
-            walk_sorted(T, o, d, max_spn, sc.node, sc.count, sc.tmin, sc.tmax, r * sc.ray_stride, sc.seg_stride, sc.cap,
-                        nk, nn);
-            nseg[r]  = nk;
-            nsamp[r] = nn;
-            if (max_per_ray) atomicMax(max_per_ray, (int32_t)nn);
-        }
+        if (l == 0) walk_ray(T, ro, rd, r, max_spn, sc, nseg, nsamp, max_per_ray);
         return;
     }
     wave_fence();
@@ -692,8 +719,9 @@ extern "C"
             TreeArgs T{pmin, pmax, flags, first_leaf(num_nodes)};
             const RayScratch sc = scratch_view(scratch, R, max_depth);
             if (R <= coop_rays(max_depth))
-                k_ray_coop<<<grid_for(R, kCoopWaves), 64 * kCoopWaves, 0, s>>>(T, ro, rd, R, max_spn, sc, ray_seg_offset,
-                                                                               ray_sample_offset, max_per_ray);
+                k_ray_coop<<<grid_for(R, kCoopWaves), 64 * kCoopWaves, 0, s>>>(T, ro, rd, R, max_spn, max_depth, sc,
+                                                                               ray_seg_offset, ray_sample_offset,
+                                                                               max_per_ray);
             else
                 k_ray_walk<<<grid_for(R, 128), 128, 0, s>>>(T, ro, rd, R, max_spn, sc, ray_seg_offset,
                                                              ray_sample_offset, max_per_ray);
