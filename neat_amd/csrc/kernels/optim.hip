@@ -83,6 +83,7 @@ __global__ void __launch_bounds__(256) k_adam(float* __restrict__ p, const float
 
 // the last-level cache of the card
 constexpr int64_t kCacheBytes = (int64_t)256 << 20;
+constexpr int64_t kAdamLaunch = (int64_t)1 << 33;  // parameters of a launch, at most
 
 }  // namespace
 }  // namespace neat
@@ -112,11 +113,16 @@ extern "C" int neat_adam_step(neat_stream_t stream, float* param, const float* g
     a.one_minus_beta2 = (float)(1.0 - beta2);
     a.eps             = (float)eps;
     a.weight_decay    = (float)weight_decay;
-    const unsigned blocks = grid_for((n + 3) / 4, 256);
-    if (16 * n > kCacheBytes)
-        k_adam<true><<<blocks, 256, 0, as_stream(stream)>>>(param, grad, exp_avg, exp_avg_sq, n, a);
-    else
-        k_adam<false><<<blocks, 256, 0, as_stream(stream)>>>(param, grad, exp_avg, exp_avg_sq, n, a);
-    NEAT_LAUNCHED();
+    // a launch holds fewer than 2^32 threads, i.e. 2^34 parameters
+    for (int64_t i = 0; i < n; i += kAdamLaunch)
+    {
+        const int64_t m       = std::min(n - i, kAdamLaunch);
+        const unsigned blocks = grid_for((m + 3) / 4, 256);
+        if (16 * n > kCacheBytes)
+            k_adam<true><<<blocks, 256, 0, as_stream(stream)>>>(param + i, grad + i, exp_avg + i, exp_avg_sq + i, m, a);
+        else
+            k_adam<false><<<blocks, 256, 0, as_stream(stream)>>>(param + i, grad + i, exp_avg + i, exp_avg_sq + i, m, a);
+        NEAT_LAUNCHED();
+    }
     return NEAT_OK;
 }

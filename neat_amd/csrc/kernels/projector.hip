@@ -1481,15 +1481,18 @@ __device__ __forceinline__ void record_sample(const ProjGeom& g, const Plan& p, 
 // Measured on 6.7 M samples of 243 k segments (FP32): 1.30 ms with one lane per segment, every channel's terms and
 // blocks in plain order; 0.78 ms with the contraction and the block order; 0.51 / 0.33 / 0.25 / 0.23 ms with 2 / 4 / 8 /
 // 16 lanes. 8, because a proposal's segments hold 8 samples.
-constexpr int kRgLanes = 8;
+// A launch takes the segments [q_begin, q_end), at most kRgLaunch: it holds fewer than 2^32 threads.
+constexpr int kRgLanes      = 8;
+constexpr int64_t kRgLaunch = (int64_t)1 << 28;
 
 template <int C, bool kBF16, bool kHalfMajor>
-__global__ void __launch_bounds__(256) k_proj_ray_grad(ProjGeom g, Plan p, const void* grid_lowp, const float* dfeat,
-                                                       float* seg_grad)
+__global__ void __launch_bounds__(256) k_proj_ray_grad(ProjGeom g, Plan p, int64_t q_begin, int64_t q_end,
+                                                       const void* grid_lowp, const float* dfeat, float* seg_grad)
 {
     const uint32_t nb8 = gridDim.x / 8;  // the grid is a multiple of 8
-    const int64_t q    = (((int64_t)(blockIdx.x % 8) * nb8 + blockIdx.x / 8) * blockDim.x + threadIdx.x) / kRgLanes;
-    if (q >= g.K) return;  // uniform over a segment's lanes
+    const int64_t t    = ((int64_t)(blockIdx.x % 8) * nb8 + blockIdx.x / 8) * blockDim.x + threadIdx.x;
+    const int64_t q    = q_begin + t / kRgLanes;
+    if (q >= q_end) return;  // uniform over a segment's lanes
     const int lq      = threadIdx.x % kRgLanes;
     const int4 ri     = p.rec_i[q];
     const int32_t k   = ri.x, n = ri.w;
@@ -1860,21 +1863,20 @@ extern "C"
             Plan p             = plan_view(ws, z);
             const float* dfeat = reinterpret_cast<const float*>(region(ws, z, 13));
             const bool bf16    = a.precision == NEAT_PREC_BF16;
-            const unsigned nb  = (grid_for(z.K * kRgLanes, 256) + 7) / 8 * 8;
-            if (z.C == 8)
+            for (int64_t q = 0; q < z.K; q += kRgLaunch)
             {
-                if (a.mfma && bf16)
-                    k_proj_ray_grad<8, true, true><<<nb, 256, 0, s>>>(a.g, p, a.grid_bf16, dfeat, seg_grad);
+                const int64_t q1  = std::min(z.K, q + kRgLaunch);
+                const unsigned nb = (grid_for((q1 - q) * kRgLanes, 256) + 7) / 8 * 8;
+                if (z.C != 8)
+                    k_proj_ray_grad<4, false, false><<<nb, 256, 0, s>>>(a.g, p, q, q1, nullptr, dfeat, seg_grad);
+                else if (a.mfma && bf16)
+                    k_proj_ray_grad<8, true, true><<<nb, 256, 0, s>>>(a.g, p, q, q1, a.grid_bf16, dfeat, seg_grad);
                 else if (a.mfma)
-                    k_proj_ray_grad<8, false, true><<<nb, 256, 0, s>>>(a.g, p, nullptr, dfeat, seg_grad);
+                    k_proj_ray_grad<8, false, true><<<nb, 256, 0, s>>>(a.g, p, q, q1, nullptr, dfeat, seg_grad);
                 else
-                    k_proj_ray_grad<8, false, false><<<nb, 256, 0, s>>>(a.g, p, nullptr, dfeat, seg_grad);
+                    k_proj_ray_grad<8, false, false><<<nb, 256, 0, s>>>(a.g, p, q, q1, nullptr, dfeat, seg_grad);
+                NEAT_LAUNCHED();
             }
-            else
-            {
-                k_proj_ray_grad<4, false, false><<<nb, 256, 0, s>>>(a.g, p, nullptr, dfeat, seg_grad);
-            }
-            NEAT_LAUNCHED();
         }
         k_ray_grad_sum<<<grid_for(R, 256), 256, 0, s>>>(x->ray_seg_offset, R, seg_grad, grad_origin,
                                                          grad_direction);
