@@ -39,6 +39,18 @@ __device__ __forceinline__ void split3(float v, __bf16 (&p)[3])
     p[2]          = (__bf16)(r - (float)p[1]);
 }
 
+// The same for any v: the first plane cut off instead of rounded, so that no finite value becomes an infinite one, and an
+// infinity or NaN in it alone.
+__device__ __forceinline__ void split3_any(float v, __bf16 (&p)[3])
+{
+    const bool nan   = v != v, finite = fabsf(v) < INFINITY;
+    const uint32_t u = (__float_as_uint(v) & 0xFFFF0000u) | (nan ? 0x400000u : 0u);
+    p[0]             = __builtin_bit_cast(__bf16, (unsigned short)(u >> 16));
+    const float r    = finite ? v - __uint_as_float(u) : 0.f;
+    p[1]             = (__bf16)r;
+    p[2]             = (__bf16)(r - (float)p[1]);
+}
+
 // the three planes of 8 values as fragments, converted two at a time
 __device__ __forceinline__ void split3_frag(const float (&v)[8], bf16x8 (&p)[3])
 {
@@ -239,6 +251,18 @@ struct SplitX
             a[j + 4] = p[1][j];
             b[j]     = p[2][j];
             b[j + 4] = p[0][j];
+        }
+    }
+    // p for values of any size
+    __device__ void split_any(const float (&x4)[4])
+    {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            __bf16 q[3];
+            split3_any(x4[j], q);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) p[k][j] = q[k];
         }
     }
 };
@@ -505,7 +529,7 @@ __device__ __forceinline__ void tile_backward_split(const float* __restrict__ pa
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const int l = threadIdx.x & 63, n = l & 31, hg = l >> 5;
     asm volatile("" ::: "memory");  // as in tile_forward_split
-    const SplitX x(x4);
+    SplitX x(x4);
     f32x16 z1[MT], z2[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) z1[mt] = split_layer1<H>(w, x, mt);
@@ -569,7 +593,11 @@ __device__ __forceinline__ void tile_backward_split(const float* __restrict__ pa
         const float t2 = fmaf(a1, t1, u8 * fmaf(a1, hmax, c1));
         // a NaN or infinity anywhere takes the plain evaluation too
         const bool clear = m1 > t1 && m2 > t2 && fabsf((x4[0] + x4[1]) + (x4[2] + x4[3])) < 1e30f && t2 < 1e30f;
-        if (__any(!clear)) tile_forward_exact<H, NEAT_ACT_RELU>(params, w, x4, beta, z1, z2);
+        if (__any(!clear))
+        {
+            tile_forward_exact<H, NEAT_ACT_RELU>(params, w, x4, beta, z1, z2);
+            x.split_any(x4);
+        }
     }
     float z = 0.f;
 #pragma unroll
