@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(kDecBwdThreads, 2) k_dec_split_bwd(const float
 }
 
 // Backward for silu on the FP32 matrix cores; one partial slice per wave (at most kDecMfmaWaves per workgroup).
-template <int H, int ACT>
+template <int H>
 __global__ void __launch_bounds__(64 * kDecMfmaWaves) k_dec_mfma_bwd(const float* __restrict__ x, int64_t S,
                                                       const float* __restrict__ params, int last_act, float beta,
                                                       const float* __restrict__ gy, float* __restrict__ gx,
@@ -162,7 +162,7 @@ __global__ void __launch_bounds__(64 * kDecMfmaWaves) k_dec_mfma_bwd(const float
         const bool valid = i < S;
         float x4[4];
         load_x4(x, i, S, x4);
-        const f32x16 dx = tile_backward_mfma<H, ACT>(w, x4, valid ? gy[i] : 0.f, valid, last_act, beta, sb, acc);
+        const f32x16 dx = tile_backward_mfma<H>(w, x4, valid ? gy[i] : 0.f, valid, last_act, beta, sb, acc);
         if (gx && valid)
         {
 #pragma unroll
@@ -301,11 +301,9 @@ extern "C"
             else if (act == NEAT_ACT_RELU)
                 k_dec_split_bwd<64><<<wg, kDecBwdThreads, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
             else if (hidden == 32)
-                k_dec_mfma_bwd<32, NEAT_ACT_SILU><<<wg, 64 * waves, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials,
-                                                                           P);
+                k_dec_mfma_bwd<32><<<wg, 64 * waves, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
             else
-                k_dec_mfma_bwd<64, NEAT_ACT_SILU><<<wg, 64 * waves, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials,
-                                                                           P);
+                k_dec_mfma_bwd<64><<<wg, 64 * waves, 0, s>>>(x, S, params, last_act, beta, gy, gx, partials, P);
             NEAT_LAUNCHED();
             k_dec_reduce_partials<<<reduce_partials_blocks(P), 256, 0, s>>>(partials, slices, P, gparams);
             NEAT_LAUNCHED();

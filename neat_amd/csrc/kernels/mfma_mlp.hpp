@@ -214,8 +214,9 @@ __device__ __forceinline__ typename P::Frag1 x_step(const float (&x4)[4], int s)
     }
 }
 
-template <typename P, int H, int ACT, typename WS>
-__device__ __forceinline__ void tile_forward_mfma(const WS& w, const float (&x4)[4], float beta, Fwd<H / 32>& f)
+template <typename P, int H>
+__device__ __forceinline__ void tile_forward_mfma(const WeightLDS<P, H>& w, const float (&x4)[4], float beta,
+                                                  Fwd<H / 32>& f)
 {
     constexpr int MT = H / 32, S = steps_per_tile<P>();
     const int l = threadIdx.x & 63, g = l >> 5;
@@ -239,7 +240,7 @@ __device__ __forceinline__ void tile_forward_mfma(const WS& w, const float (&x4)
 #pragma unroll
             for (int st = 0; st < S; ++st)
             {
-                auto b = P::from_acc(f.z1[ms], st, [&](float v, int) { return act_f(ACT, v, beta); });
+                auto b = P::from_acc(f.z1[ms], st, [&](float v, int) { return act_f(NEAT_ACT_SILU, v, beta); });
                 acc    = P::mma(w.w2[mt][ms][st][l], b, acc);
             }
         }
@@ -252,7 +253,7 @@ __device__ __forceinline__ void tile_forward_mfma(const WS& w, const float (&x4)
     for (int mt = 0; mt < MT; ++mt)
     {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) part = fmaf(w.vec[2][32 * mt + crow(i, g)], act_f(ACT, f.z2[mt][i], beta), part);
+        for (int i = 0; i < 16; ++i) part = fmaf(w.vec[2][32 * mt + crow(i, g)], act_f(NEAT_ACT_SILU, f.z2[mt][i], beta), part);
     }
     f.z = part + __shfl_xor(part, 32) + w.vec[3][0];
 }
@@ -330,11 +331,11 @@ struct BwdAcc
     }
 };
 
-// FP32 backward of one tile of 32 samples on a wave: recompute the forward (tile_forward_mfma), take dz = gy *
+// FP32 backward (silu) of one tile of 32 samples on a wave: recompute the forward (tile_forward_mfma), take dz = gy *
 // last_act'(z) (0 for invalid lanes), back-propagate on the matrix cores, and add the tile's parameter-gradient
 // products to acc (products over the tile's samples, staged through LDS as [row][sample]). Returns dL/dx in
 // registers 0..3 of each lane (channels 4g..4g+3 of its sample, g = lane / 32).
-template <int H, int ACT>
+template <int H>
 __device__ __forceinline__ f32x16 tile_backward_mfma(const WeightLDS<PrecF32, H>& w, const float (&x4)[4], float gy,
                                                      bool valid, int last_act, float beta, const BwdStage<H>& sb,
                                                      BwdAcc<H / 32>& acc)
@@ -345,7 +346,7 @@ __device__ __forceinline__ f32x16 tile_backward_mfma(const WeightLDS<PrecF32, H>
     constexpr int KSTEPS = 32 / (2 * P::KS);  // sample steps of a weight-gradient product
     const int l = threadIdx.x & 63, n = l & 31, hg = l >> 5;
     Fwd<MT> f;
-    tile_forward_mfma<P, H, ACT>(w, x4, beta, f);
+    tile_forward_mfma<P, H>(w, x4, beta, f);
     const float dz = valid ? gy * act_d(last_act, f.z, beta) : 0.f;
     if (hg == 0) acc.b3 += dz;
     // X tile and the first staged pair: dZ2 (A) and act(z1) (B)
@@ -360,9 +361,9 @@ __device__ __forceinline__ f32x16 tile_backward_mfma(const WeightLDS<PrecF32, H>
         for (int i2 = 0; i2 < 16; ++i2)
         {
             const int r = 32 * mt + crow(i2, hg);
-            dZ2[mt][i2] = w.vec[2][r] * dz * act_d(ACT, f.z2[mt][i2], beta);
+            dZ2[mt][i2] = w.vec[2][r] * dz * act_d(NEAT_ACT_SILU, f.z2[mt][i2], beta);
             ST::put(sb.sA, r, n, dZ2[mt][i2]);
-            ST::put(sb.sB, r, n, act_f(ACT, f.z1[mt][i2], beta));
+            ST::put(sb.sB, r, n, act_f(NEAT_ACT_SILU, f.z1[mt][i2], beta));
         }
     }
     wave_lds_fence();
@@ -389,7 +390,7 @@ __device__ __forceinline__ f32x16 tile_backward_mfma(const WeightLDS<PrecF32, H>
     for (int mt = 0; mt < MT; ++mt)
     {
 #pragma unroll
-        for (int i2 = 0; i2 < 16; ++i2) ST::put(sb.sB, 32 * mt + crow(i2, hg), n, act_f(ACT, f.z2[mt][i2], beta));
+        for (int i2 = 0; i2 < 16; ++i2) ST::put(sb.sB, 32 * mt + crow(i2, hg), n, act_f(NEAT_ACT_SILU, f.z2[mt][i2], beta));
     }
     wave_lds_fence();
 #pragma unroll
@@ -413,7 +414,7 @@ __device__ __forceinline__ f32x16 tile_backward_mfma(const WeightLDS<PrecF32, H>
                 a = P::mma(w.w2t[mt][ms][st][l], P::from_acc(dZ2[ms], st, [](float v, int) { return v; }), a);
         }
 #pragma unroll
-        for (int i2 = 0; i2 < 16; ++i2) a[i2] *= act_d(ACT, f.z1[mt][i2], beta);
+        for (int i2 = 0; i2 < 16; ++i2) a[i2] *= act_d(NEAT_ACT_SILU, f.z1[mt][i2], beta);
         dZ1[mt] = a;
     }
     // dL/dx: rows 0..7 of W0^T dZ1, i.e. registers 0..3 of each lane group (channels 4g..4g+3)

@@ -903,12 +903,6 @@ __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const floa
     BwdAcc<MT> acc;
     float amax = 0.f;  // largest |dL/dfeature| this lane wrote
     const int64_t nchunks = p.chunk_off1[g.N];
-    // the chunk's largest |dL/dfeature| into its slot's entry (dmax[1 + slot])
-    auto slot_max = [&](float m, int32_t slot) {
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-        if (l == 0) atomicMax(dmax + 1 + slot, __float_as_uint(m));
-    };
     for (int64_t c = blockIdx.x; c < nchunks; c += gridDim.x)
     {
         const int32_t slot = p.chunk1_slot[c];
@@ -922,7 +916,6 @@ __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const floa
         const void* ngrid = node_grid_ptr(g, nullptr, false, slot);
         __syncthreads();
         const int32_t nsamp = cx.beg[nseg];
-        float cmax = 0.f;  // this chunk's
         for (int32_t w0 = 0; w0 < nsamp; w0 += kFwdChunk)
         {
             const int32_t wn = min(kFwdChunk, nsamp - w0);
@@ -931,13 +924,13 @@ __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const floa
             // pairs of tiles per wave (fetch_pair)
             auto tile = [&](int32_t i, const float (&x4)[4], float gy) {
                 const bool valid = i < wn;
-                const f32x16 dx = tile_backward_mfma<H, NEAT_ACT_SILU>(w, x4, gy, valid, NEAT_ACT_SOFTPLUS, g.beta, sb, acc);
+                const f32x16 dx = tile_backward_mfma<H>(w, x4, gy, valid, NEAT_ACT_SOFTPLUS, g.beta, sb, acc);
                 if (valid)
                 {
                     // [2][S][4]: channel halves
                     *reinterpret_cast<float4*>(dfeat + ((int64_t)hg * g.S + base + w0 + i) * 4) =
                         make_float4(dx[0], dx[1], dx[2], dx[3]);
-                    cmax = fmaxf(cmax, fmaxf(fmaxf(fabsf(dx[0]), fabsf(dx[1])), fmaxf(fabsf(dx[2]), fabsf(dx[3]))));
+                    amax = fmaxf(amax, fmaxf(fmaxf(fabsf(dx[0]), fabsf(dx[1])), fmaxf(fabsf(dx[2]), fabsf(dx[3]))));
                 }
             };
             for (int32_t p0 = wave * 64; p0 < wn; p0 += 256)
@@ -957,8 +950,6 @@ __global__ void __launch_bounds__(256) k_mfma_bwd(ProjGeom g, Plan p, const floa
             }
             __syncthreads();
         }
-        slot_max(cmax, slot);
-        amax = fmaxf(amax, cmax);
     }
     // this wave's slice of the partial parameter gradient (packed layout)
     write_param_partials<H, C>(acc, partials + ((int64_t)blockIdx.x * 4 + wave) * P_total);

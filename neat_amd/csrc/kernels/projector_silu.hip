@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(kBf16FwdThreads, 3) k_bf16_fwd(ProjGeom g, Pla
 #pragma unroll
                     for (int j = 0; j < 4; ++j) x[j] = h ? cur.xb[j] : cur.xa[j];
                     Fwd<H / 32> f;
-                    tile_forward_mfma<PrecBF16, H, NEAT_ACT_SILU>(w, x, g.beta, f);
+                    tile_forward_mfma<PrecBF16, H>(w, x, g.beta, f);
                     z[0] = h ? z[0] : f.z;
                     z[1] = h ? f.z : z[1];
                 }

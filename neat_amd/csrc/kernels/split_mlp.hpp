@@ -197,8 +197,8 @@ __device__ __forceinline__ f32x16 row_vec(const float* v, int mt, int g)
     return r;
 }
 
-// The pre-activations of both hidden layers as tile_forward_mfma<PrecF32, H, ACT> computes them, bit for bit,
-// the weights read from global memory (row crow(4q, g).. of a fragment are 4 consecutive floats).
+// The pre-activations of both hidden layers in the steps of tile_forward_mfma<PrecF32, H>, plain FP32 matrix products, the
+// weights read from global memory (row crow(4q, g).. of a fragment are 4 consecutive floats).
 template <int H, int ACT>
 __device__ __forceinline__ void tile_forward_exact(const float* __restrict__ params, const WeightLDSSplitFwd<H>& w,
                                                    const float (&x4)[4], float beta, f32x16 (&z1)[H / 32],
