@@ -350,9 +350,9 @@ __global__ void __launch_bounds__(64 * kCoopWaves) k_ray_coop(TreeArgs T, const 
 {
     if (!exact_boxes(T, max_depth))
     {
-        // the grid has 64 times the threads this takes
-        const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-        if (r < R) walk_ray(T, ro, rd, r, max_spn, sc, nseg, nsamp, max_per_ray);
+        // one wave's rays to a workgroup (the grid has 64 times the threads this takes): they spread over more CUs
+        const int64_t r = (int64_t)blockIdx.x * 64 + threadIdx.x;
+        if (threadIdx.x < 64 && r < R) walk_ray(T, ro, rd, r, max_spn, sc, nseg, nsamp, max_per_ray);
         return;
     }
     __shared__ CoopList s_list[kCoopWaves][2];

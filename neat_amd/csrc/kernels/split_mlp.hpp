@@ -599,12 +599,9 @@ __device__ __forceinline__ void tile_backward_split(const float* __restrict__ pa
         const float t1 = u8 * fmaf(a0, max_abs_x(x4), c0);
         const float t2 = fmaf(a1, t1, u8 * fmaf(a1, hmax, c1));
         // a NaN or infinity anywhere takes the plain evaluation too
-        const bool clear = m1 > t1 && m2 > t2 && fabsf((x4[0] + x4[1]) + (x4[2] + x4[3])) < 1e30f && t2 < 1e30f;
-        if (__any(!clear))
-        {
-            tile_forward_exact<H, NEAT_ACT_RELU>(params, w, x4, beta, z1, z2);
-            x.split_any(x4);
-        }
+        const bool fine = fabsf((x4[0] + x4[1]) + (x4[2] + x4[3])) < 1e30f && t2 < 1e30f;
+        if (__any(!(fine && m1 > t1 && m2 > t2))) tile_forward_exact<H, NEAT_ACT_RELU>(params, w, x4, beta, z1, z2);
+        if (__any(!fine)) x.split_any(x4);
     }
     float z = 0.f;
 #pragma unroll
