@@ -6,7 +6,7 @@
 // in LDS. The forward and the relu backward take their products in split form on the BF16 matrix cores (split_mlp.hpp),
 // the silu backward on the FP32 ones (v_mfma_f32_32x32x2f32, the tiles of mfma_mlp.hpp). Other shapes run the
 // vector-ALU tiles of mlp_tile.hpp, one wave per tile of 64 samples. On 10^6 rows with H = 64, relu, forward and
-// backward took 112 and 484 us on the FP32 matrix cores and take 55 and 150 us in split form.
+// backward take 103 and 456 us on the FP32 matrix cores and 58 and 191 us in split form (calls, one after the other).
 //
 // Backward (all forms): each wave or workgroup recomputes its tiles' forward, back-propagates, and accumulates its
 // share of the parameter gradient into its own slice of a partials buffer (every entry written by one thread); a

@@ -3,10 +3,11 @@
 //
 // On the FP32 matrix cores a tile of 32 samples with H = 64 took 4,608 cycles of products forward and 21,000 backward
 // (a 32x32x2 product is 64 cycles); in split form it is 1,730 and 4,160, beside about 2,200 and 5,900 cycles of vector
-// work. Measured on 53.3 M samples (2^18 rays, 4096 grids of 17^3 x 8): forward 7.37 -> 3.5 ms, backward 28.3 -> 8.3 ms
-// (10.9 with every pre-activation recomputed on the FP32 matrix cores; 0.5 ms are the tiles that are). The gather of
-// the node grid takes about 1.3 ms of the backward; two waves per SIMD leave the matrix cores idle two thirds of the
-// time, the rest being vector work and exposed LDS latency.
+// work. Measured on 53.3 M samples (2^18 rays, 4096 grids of 17^3 x 8): forward 7.37 -> 3.6 ms, backward 28.3 -> 9.2 ms
+// (0.5 ms are the tiles whose pre-activations are recomputed on the FP32 matrix cores, all of them would cost 2.5 ms
+// more; 0.9 ms the order of the sums and the output weights' own, see split_mlp.hpp). The gather of the node grid takes
+// about 1.3 ms of the backward; two waves per SIMD leave the matrix cores idle two thirds of the time, the rest being
+// vector work and exposed LDS latency.
 #include "projector_dev.hpp"
 #include "split_mlp.hpp"
 
