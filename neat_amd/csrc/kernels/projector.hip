@@ -1029,21 +1029,27 @@ SortShape sort_shape(int64_t K, int64_t N)
 size_t sort_items_bytes(int64_t K) { return (4 * (size_t)K + 255) / 256 * 256; }
 size_t sort_counts_bytes(const SortShape& q) { return (8 * (size_t)(q.tiles * q.bins + 1) + 255) / 256 * 256; }
 
+// The temporary storage grows with K and N across the rule of own_sort, so that a workspace sized for a program's largest
+// batch and tree serves its smaller ones: the counting sorts' at 256 digits (about 9 B an item) whatever N, and no less than
+// that where the library's radix sort is taken (about 8 B an item, and up to 4096 items less than the former's for 4097).
+size_t sort_temp_bytes(int64_t K, int64_t N)
+{
+    const int64_t counts = (K + kSortTile - 1) / kSortTile * kSortBins;
+    const size_t own     = 2 * sort_items_bytes(K) + (8 * (size_t)(counts + 1) + 255) / 256 * 256 +
+                       scan_workspace_bytes(counts + 1);
+    if (own_sort(K, N)) return own;
+    size_t lib = 0;
+    hipcub::DeviceRadixSort::SortPairs(nullptr, lib, (int32_t*)nullptr, (int32_t*)nullptr, (int32_t*)nullptr,
+                                       (int32_t*)nullptr, (int)std::max<int64_t>(K, 1), 0, 32);
+    return std::max(own, lib);
+}
+
 ProjSizes proj_sizes(int64_t K, int64_t S, int64_t N, int32_t G, int32_t C, int32_t P, bool prop)
 {
     ProjSizes z{K, S, N, G, C, P, 0, 0, scatter_chunk(S), 0, prop};
     z.max1 = (S + (int64_t)kSegCost * K + kFwdChunk - 1) / kFwdChunk + N;
     z.max2 = (S + z.chunk2 - 1) / z.chunk2 + N;
-    if (own_sort(K, N))
-    {
-        const SortShape q = sort_shape(K, N);
-        z.sort_temp       = 2 * sort_items_bytes(K) + sort_counts_bytes(q) + scan_workspace_bytes(q.tiles * q.bins + 1);
-        return z;
-    }
-    size_t tmp = 0;
-    hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, (int32_t*)nullptr, (int32_t*)nullptr, (int32_t*)nullptr,
-                                       (int32_t*)nullptr, (int)std::max<int64_t>(K, 1), 0, 32);
-    z.sort_temp = tmp;
+    z.sort_temp = sort_temp_bytes(K, N);
     return z;
 }
 
