@@ -829,13 +829,15 @@ extern "C"
     {
         NEAT_REQUIRE(R >= 0 && ray_seg_offset && ray_sample_offset && totals, "neat_raysample_totals: bad arguments");
         hipPointerAttribute_t at;
-        if (hipPointerGetAttributes(&at, totals) != hipSuccess || at.type != hipMemoryTypeHost)
+        if (hipPointerGetAttributes(&at, totals) != hipSuccess || at.type != hipMemoryTypeHost || !at.devicePointer)
         {
             (void)hipGetLastError();
             return fail(NEAT_E_ARG, "neat_raysample_totals: totals must be pinned host memory");
         }
         hipStream_t s = as_stream(stream);
-        k_ray_totals<<<1, 1, 0, s>>>(ray_seg_offset, ray_sample_offset, max_per_ray, R, totals);
+        // the device's address of it, which for registered memory is another than the host's
+        k_ray_totals<<<1, 1, 0, s>>>(ray_seg_offset, ray_sample_offset, max_per_ray, R,
+                                     static_cast<int64_t*>(at.devicePointer));
         NEAT_LAUNCHED();
         NEAT_HIP(hipStreamSynchronize(s));
         return NEAT_OK;
