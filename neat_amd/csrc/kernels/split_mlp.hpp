@@ -505,7 +505,9 @@ __device__ __forceinline__ void transpose_step(float* v)
 }
 
 // The sum of value j = n / (32 / N) over the 32 lanes of each half wave, on lane n of the half, of N = 16 or 32 values per
-// lane: halving the values in every step takes about 3 N instructions, the N sums one by one 5 N.
+// lane: halving the values in every step takes about 3 N instructions, the N sums one by one 5 N. The steps are taken to
+// the end for every tile, so that a lane keeps one running sum: with 4, 8 or 16 of them and the last steps once at the end
+// the projector's FP32 step takes 15.5, 17.0 and 19.3 ms instead of 15.0 (registers).
 template <int N>
 __device__ __forceinline__ float transpose_sum(float (&v)[N])
 {
